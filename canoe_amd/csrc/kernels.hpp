@@ -629,11 +629,6 @@ __device__ inline void flux_jac(double gm1, const double* w, Mt<B>& out) {
       out.a[a][c] = d[(B == 5) ? a : id3[a]][(B == 5) ? c : id3[c]];
 }
 
-struct KImplicit {
-  double dt;
-  long long ncol;  // interior columns nx2 nx3
-};
-
 // |A| at a face, evaluated with the zero/one structure of R and R^-1 of
 // flux_decomposition.hpp:91-98 spelled out (terms whose factor is an exact
 // zero are dropped, unit factors taken exactly) and fused multiply-adds.
@@ -956,41 +951,6 @@ __device__ __forceinline__ bool fwd_column(const KGrid& g, const KThermo& th,
   return ok;
 }
 
-template <int NM, int B>
-__global__ void __launch_bounds__(64)
-    k_implicit_fwd(KGrid g, KThermo th, KImplicit ip,
-                   const double* __restrict__ w, const double* __restrict__ du,
-                   double* __restrict__ arch, int* __restrict__ status) {
-  long long col = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (col >= ip.ncol) return;
-  int j = g.js + (int)(col % g.nx2);
-  int k = g.ks + (int)(col / g.nx2);
-  if (!fwd_column<NM, B>(g, th, ip.dt, w, du, g.at(0, k, j, 0), arch, ip.ncol, col))
-    atomicOr(status, 1);
-}
-
-// delta_i of the back substitution (forward_backward.hpp:86-97): level i
-// from the archive and delta_{i+1}.
-template <int B>
-__device__ inline void back_step(const double* __restrict__ arch,
-                                 long long lb, long long as, long long ao,
-                                 bool top, const Vt<B>& dn, Vt<B>& d) {
-#pragma unroll
-  for (int r = 0; r < B; ++r) d.v[r] = __builtin_nontemporal_load(&arch[(lb + B * B + r) * as + ao]);
-  if (!top) {
-    Mt<B> a;
-#pragma unroll
-    for (int r = 0; r < B; ++r)
-#pragma unroll
-      for (int q = 0; q < B; ++q)
-        a.a[r][q] = __builtin_nontemporal_load(&arch[(lb + r * B + q) * as + ao]);
-    Vt<B> ad;
-    mvec<B>(a, dn, ad);
-#pragma unroll
-    for (int r = 0; r < B; ++r) d.v[r] = d.v[r] - ad.v[r];
-  }
-}
-
 // Write-back of the solution into a cell's du (forward_backward.hpp:221-246:
 // the total-density increment is split over the species by w_n).
 template <int NM, int B>
@@ -1018,39 +978,6 @@ __device__ inline void write_back(const Vt<B>& d, const double* duo,
 #pragma unroll
   for (int n = 1; n < IVX; ++n) d0 -= dun[n];
   dun[0] = d0;
-}
-
-// Back substitution writing du in place (cg_implicit_solve).
-template <int NM, int B>
-__global__ void __launch_bounds__(64)
-    k_implicit_bwd(KGrid g, KImplicit ip, const double* __restrict__ w,
-                   const double* __restrict__ arch, double* __restrict__ du) {
-  constexpr int N = 5 + NM;
-  constexpr int AS = B * B + B;
-  long long col = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (col >= ip.ncol) return;
-  int j = g.js + (int)(col % g.nx2);
-  int k = g.ks + (int)(col / g.nx2);
-  const int is = g.is, ie = g.ie;
-  const long long c0 = g.at(0, k, j, 0);
-  const long long sn = g.c.n, si = g.c.i;
-  Vt<B> dn;
-  for (int i = ie; i >= is; --i) {
-    Vt<B> d;
-    back_step<B>(arch, (long long)(i - is) * AS, ip.ncol, col, i == ie, dn, d);
-    dn = d;
-    const long long ci = c0 + i * si;
-    double duo[N], wsp[N], dun[N];
-#pragma unroll
-    for (int n = 0; n < N; ++n) {
-      duo[n] = (NM > 0 || n >= 1 + NM) ? du[ci + n * sn] : 0.0;
-      wsp[n] = (n >= 1 && n <= NM) ? w[ci + n * sn] : 0.0;
-    }
-    if (NM == 0) duo[0] = du[ci];
-    write_back<NM, B>(d, duo, wsp, dun);
-#pragma unroll
-    for (int n = 0; n < N; ++n) du[ci + n * sn] = dun[n];
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1417,22 +1344,6 @@ __device__ __forceinline__ void bwd_update_column(
     }
   }
   (void)rtop;
-}
-
-template <int NM, int B>
-__global__ void __launch_bounds__(64)
-    k_implicit_bwd_update(KGrid g, KThermo th, KImplicit ip, KUpdate up,
-                          const double* __restrict__ arch,
-                          const double* __restrict__ du, double* __restrict__ u,
-                          double* __restrict__ u1, double* __restrict__ w,
-                          double* __restrict__ psf, double* __restrict__ psv,
-                          int* __restrict__ status) {
-  long long col = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (col >= ip.ncol) return;
-  int j = g.js + (int)(col % g.nx2);
-  int k = g.ks + (int)(col / g.nx2);
-  bwd_update_column<NM, B>(g, th, up, arch, ip.ncol, col, du, u, u1, w, psf, psv,
-                           g.at(0, k, j, 0), col * g.ps_c, status);
 }
 
 // ---------------------------------------------------------------------------

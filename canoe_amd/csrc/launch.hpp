@@ -10,7 +10,7 @@
 #include "flux32.hpp"
 #include "kernels.hpp"
 #include "kessler.hpp"
-#include "lines.hpp"
+#include "rows.hpp"
 
 namespace cg_host {
 using namespace cg;
@@ -151,43 +151,6 @@ void launch_fluxes(const KGrid& g, const KThermo& th, const cg_config& cfg,
   }
 }
 
-template <int NM>
-void launch_implicit(const KGrid& g, const KThermo& th, double dt, int flag,
-                     double* du, const double* w, double* arch, int* status,
-                     hipStream_t s, KTimer* tm = nullptr) {
-  KImplicit ip;
-  ip.dt = dt;
-  ip.ncol = (long long)g.nx2 * g.nx3;
-  unsigned nb = nblk(ip.ncol, 64);
-  if (flag & 8) {
-    TIMED(tm, KID_IMPLICIT_FWD,
-          (k_implicit_fwd<NM, 5><<<nb, 64, 0, s>>>(g, th, ip, w, du, arch, status)));
-    TIMED(tm, KID_IMPLICIT_BWD,
-          (k_implicit_bwd<NM, 5><<<nb, 64, 0, s>>>(g, ip, w, arch, du)));
-  } else {
-    TIMED(tm, KID_IMPLICIT_FWD,
-          (k_implicit_fwd<NM, 3><<<nb, 64, 0, s>>>(g, th, ip, w, du, arch, status)));
-    TIMED(tm, KID_IMPLICIT_BWD,
-          (k_implicit_bwd<NM, 3><<<nb, 64, 0, s>>>(g, ip, w, arch, du)));
-  }
-}
-
-template <int NM>
-void launch_bc(const KGrid& g, double* w, hipStream_t s, KTimer* tm = nullptr) {
-  TIMED(tm, KID_BC_X1,
-        (k_bc_x1<NM><<<nblk((long long)g.nx2 * g.nx3 * NG, 256), 256, 0, s>>>(g, w)));
-  if (g.f2)
-    TIMED(tm, KID_BC_X2,
-          (k_bc_x2<NM><<<nblk((long long)g.nc1 * g.nx3 * NG, 256), 256, 0, s>>>(g, w)));
-  if (g.f3)
-    TIMED(tm, KID_BC_X3,
-          (k_bc_x3<NM><<<nblk((long long)g.nc1 * g.nc2 * NG, 256), 256, 0, s>>>(g, w)));
-}
-
-inline size_t arch_doubles(const KGrid& g) {
-  return (size_t)g.nx1 * 30 * (size_t)g.nx2 * g.nx3;
-}
-
 // The lines of direction dir (0 = x1, 1 = x2, 2 = x3) of a block: lanes
 // along the transverse index of smaller stride; Cartesian face areas and
 // volume (x1 faces dx2 dx3, x2 faces dx1 dx3, x3 faces dx1 dx2).
@@ -225,6 +188,55 @@ inline KLines make_lines(const KGrid& g, int dir) {
   return L;
 }
 
+// Eight lanes per line where the lines are few.  A round of 8,192 lines (8 per
+// wavefront, a wavefront per SIMD of 256 compute units) takes about 2.2 us
+// per level, the one-lane kernels 5.5 us per level for any number of lines
+// up to 65,536 and then their memory time (5 x 5 blocks, stage of a run, 128
+// levels: 9,216 columns 0.54 against 0.72 ms, 16,384 columns 0.66 against
+// 0.74, 25,600 columns 1.17 against 0.84; 3 x 3: 9,216 columns 0.29 against
+// 0.40, 16,384 columns 0.42 against 0.41): two rounds.
+constexpr long long ROWS_MAX_LINES = 16384;
+
+inline unsigned rows_grid(long long nline) { return nblk(nline, RLINES * RWAVES); }
+
+// The x1 columns of caller arrays, eight lanes per column at every size: in
+// the AthenaArray layout its lanes run along the column (64 bytes per octet),
+// where one lane per column put every lane of a load on a cache line of its
+// own.  256 x 256 columns of 128 levels: 2.08 ms against 2.58 (5 x 5), 1.12
+// against 2.18 ms (3 x 3); 32 x 32 columns of 128 levels 0.19 ms.
+template <int NM>
+void launch_implicit(const KGrid& g, const KThermo& th, double dt, int flag,
+                     double* du, const double* w, double* arch, int* status,
+                     hipStream_t s, KTimer* tm = nullptr) {
+  const long long ncol = (long long)g.nx2 * g.nx3;
+  const bool flo = g.bc[0] != CG_BC_PERIODIC, fhi = g.bc[1] != CG_BC_PERIODIC;
+  const KLines L = make_lines(g, 0);
+  if (flag & 8)
+    TIMED(tm, KID_IMPLICIT_FUSED,
+          (k_rows_walls<NM, 5, 0><<<rows_grid(ncol), 64 * RWAVES, 0, s>>>(
+              L, th, dt, nullptr, flo, fhi, w, du, arch, status)));
+  else
+    TIMED(tm, KID_IMPLICIT_FUSED,
+          (k_rows_walls<NM, 3, 0><<<rows_grid(ncol), 64 * RWAVES, 0, s>>>(
+              L, th, dt, nullptr, flo, fhi, w, du, arch, status)));
+}
+
+template <int NM>
+void launch_bc(const KGrid& g, double* w, hipStream_t s, KTimer* tm = nullptr) {
+  TIMED(tm, KID_BC_X1,
+        (k_bc_x1<NM><<<nblk((long long)g.nx2 * g.nx3 * NG, 256), 256, 0, s>>>(g, w)));
+  if (g.f2)
+    TIMED(tm, KID_BC_X2,
+          (k_bc_x2<NM><<<nblk((long long)g.nc1 * g.nx3 * NG, 256), 256, 0, s>>>(g, w)));
+  if (g.f3)
+    TIMED(tm, KID_BC_X3,
+          (k_bc_x3<NM><<<nblk((long long)g.nc1 * g.nc2 * NG, 256), 256, 0, s>>>(g, w)));
+}
+
+inline size_t arch_doubles(const KGrid& g) {
+  return (size_t)g.nx1 * 30 * (size_t)g.nx2 * g.nx3;
+}
+
 // Scratch doubles of the line solve of direction dir (B x B blocks).
 inline size_t line_doubles(const KGrid& g, int dir, int B, bool per) {
   KLines L = make_lines(g, dir);
@@ -237,7 +249,11 @@ void launch_lines_d(const KLines& L, const KThermo& th, double dt, const double*
                     bool per, double* du, const double* w, double* lv, int* status,
                     hipStream_t s, KTimer* tm) {
   const unsigned nb = nblk(L.nline, 64);
-  if (per)
+  if (!per && L.nline <= ROWS_MAX_LINES)
+    TIMED(tm, KID_LINES,
+          (k_rows_walls<NM, B, DIR><<<rows_grid(L.nline), 64 * RWAVES, 0, s>>>(
+              L, th, dt, dtp, true, true, w, du, lv, status)));
+  else if (per)
     TIMED(tm, KID_LINES,
           (k_line_periodic<NM, B, DIR><<<nb, 64, 0, s>>>(L, th, dt, dtp, w, du, lv, status)));
   else

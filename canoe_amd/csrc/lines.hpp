@@ -230,24 +230,49 @@ struct LineAsm {
 // 216-229), species unchanged.  x2 / x3 lines store IDN, the normal momentum
 // and IEN only, the variables the reference copies out of its line buffer
 // (solve_implicit_3d.cpp:51-56, 82-87).
+// The cell's du and the species weights are loaded apart (LineCell).
+template <int NM, int DIR>
+struct LineCell {
+  static constexpr int N = 5 + NM, IVX = 1 + NM;
+  double o[N], ws[N];
+  // walls: the species weights are needed
+  __device__ __forceinline__ void load(const KLines& L, const double* __restrict__ w,
+                                       const double* __restrict__ du, long long org, long long t,
+                                       int i, bool walls) {
+    const long long ci = org + (long long)i * L.sl;
+#pragma unroll
+    for (int n = 0; n < N; ++n) o[n] = du[ci + n * L.sn];
+#pragma unroll
+    for (int n = 1; n < IVX; ++n)
+      ws[n] = !walls ? 0.0
+                     : (DIR == 0 ? w[ci + n * L.sn] : w_shuffled<DIR>(L, w, n, t, i));
+  }
+  // the loads are waited for here (and not together with later stores)
+  __device__ __forceinline__ void land() {
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      asm volatile("" : "+v"(o[n]));
+      if (n >= 1 && n < IVX) asm volatile("" : "+v"(ws[n]));
+    }
+  }
+};
+
 template <int NM, int B, int DIR, bool PER>
-__device__ inline void line_write_back(const Vt<B>& d, const double* __restrict__ w,
-                                       double* __restrict__ du, long long ci,
-                                       long long sn, const KLines& L, long long t,
-                                       int i) {
+__device__ __forceinline__ void line_store(const Vt<B>& d, const LineCell<NM, DIR>& c,
+                                           double* __restrict__ du, long long ci,
+                                           long long sn) {
   constexpr int N = 5 + NM, IVX = 1 + NM, IEN = 4 + NM;
   constexpr int vn = IVX + DIR, vt1 = IVX + (1 + DIR) % 3, vt2 = IVX + (2 + DIR) % 3;
   double o[N];
 #pragma unroll
-  for (int n = 0; n < N; ++n) o[n] = du[ci + n * sn];
+  for (int n = 0; n < N; ++n) o[n] = c.o[n];
   if (!PER) {
     double dens = o[0];
 #pragma unroll
     for (int n = 1; n < IVX; ++n) dens += o[n];
     dens = d.v[0] - dens;
 #pragma unroll
-    for (int n = 1; n < IVX; ++n)
-      o[n] += dens * (DIR == 0 ? w[ci + n * sn] : w_shuffled<DIR>(L, w, n, t, i));
+    for (int n = 1; n < IVX; ++n) o[n] += dens * c.ws[n];
   }
   o[0] = d.v[0];
   if (B == 5) {
@@ -269,6 +294,15 @@ __device__ inline void line_write_back(const Vt<B>& d, const double* __restrict_
     du[ci + vn * sn] = o[vn];
     du[ci + IEN * sn] = o[IEN];
   }
+}
+
+template <int NM, int B, int DIR, bool PER>
+__device__ inline void line_write_back(const Vt<B>& d, const double* __restrict__ w,
+                                       double* __restrict__ du, long long org,
+                                       const KLines& L, long long t, int i) {
+  LineCell<NM, DIR> c;
+  c.load(L, w, du, org, t, i, !PER);
+  line_store<NM, B, DIR, PER>(d, c, du, org + (long long)i * L.sl, L.sn);
 }
 
 // Gauss-Jordan elimination of [M | C | t] with partial pivoting (first row
@@ -419,8 +453,7 @@ __global__ void __launch_bounds__(64)
       for (int r = 0; r < B; ++r) d.v[r] = d.v[r] - ad.v[r];
     }
     dn = d;
-    line_write_back<NM, B, DIR, false>(d, w, du, o + (long long)(lo + p) * L.sl, L.sn,
-                                       L, t, lo + p);
+    line_write_back<NM, B, DIR, false>(d, w, du, o, L, t, lo + p);
   }
 }
 
@@ -588,8 +621,7 @@ __global__ void __launch_bounds__(64)
     mvec<B>(ai, z, xl);
   }
   if (!ok) atomicOr(status, 1);
-  line_write_back<NM, B, DIR, true>(xl, w, du, o + (long long)(lo + n - 1) * L.sl, L.sn,
-                                    L, t, lo + n - 1);
+  line_write_back<NM, B, DIR, true>(xl, w, du, o, L, t, lo + n - 1);
   Vt<B> xn = xl;
   Mt<B> zero;
 #pragma unroll
@@ -612,8 +644,7 @@ __global__ void __launch_bounds__(64)
     for (int r = 0; r < B; ++r) tv.v[r] = (cur[(OZ + r) * st] - ux.v[r]) - gx.v[r];
     mvec<B>(ai, tv, x);
     xn = x;
-    line_write_back<NM, B, DIR, true>(x, w, du, o + (long long)(lo + p) * L.sl, L.sn, L,
-                                      t, lo + p);
+    line_write_back<NM, B, DIR, true>(x, w, du, o, L, t, lo + p);
   }
 }
 

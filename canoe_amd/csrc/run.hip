@@ -127,11 +127,28 @@ unsigned implicit_grid(const cg_run* r) {
   return (unsigned)std::max(1LL, std::min(g, full));
 }
 
+// The default launch shape of the column solve takes eight lanes per column
+// where the run has few of them (ROWS_MAX_LINES); any other shape, and every
+// autotune candidate but the default, is the one-lane kernel it names.
+bool rows_columns(const cg_run* r) {
+  return r->tune.implicit_wpb == 1 && r->tune.implicit_grid == 0 && r->tune.implicit_fused &&
+         r->ngroups * 64LL <= ROWS_MAX_LINES;
+}
+
 // beta: the stage weight; the sweep's step is beta times the device step.
 template <int NM, int B, int WPB, bool KES>
 void launch_col_batch(cg_run* r, double beta, const KUpdate& up, KTimer* tm) {
   hipStream_t s = r->ctx->stream;
   const unsigned gr = implicit_grid(r);
+  if constexpr (!KES)
+    if (rows_columns(r)) {
+      TIMED(tm, KID_IMPLICIT_FUSED,
+            (k_rows_update_batch<NM, B><<<nblk((long long)r->ngroups * 64, RLINES * RWAVES),
+                                          64 * RWAVES, 0, s>>>(
+                r->d_bp, r->d_grp, r->ngroups, r->kt, beta, r->d_dt, up, r->arch,
+                r->ctx->d_status)));
+      return;
+    }
   if (r->tune.implicit_fused) {
     if constexpr (KES)
       TIMED(tm, KID_IMPLICIT_FUSED,
