@@ -12,6 +12,10 @@
 
 namespace cg {
 
+// The loads of v are waited for here, so that a later wait need not include
+// the stores issued in between.
+__device__ __forceinline__ void landed(double& v) { asm volatile("" : "+v"(v)); }
+
 // check_reconstruct (src/checks.cpp:79-97), run after the face states of
 // every direction are reconstructed (patches/19.calculate_fluxes.patch:45,
 // 73, 117): a negative face density or pressure (pb + the stored pressure,

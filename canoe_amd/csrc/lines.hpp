@@ -251,8 +251,8 @@ struct LineCell {
   __device__ __forceinline__ void land() {
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      asm volatile("" : "+v"(o[n]));
-      if (n >= 1 && n < IVX) asm volatile("" : "+v"(ws[n]));
+      landed(o[n]);
+      if (n >= 1 && n < IVX) landed(ws[n]);
     }
   }
 };

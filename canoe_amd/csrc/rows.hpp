@@ -54,10 +54,6 @@ __device__ __forceinline__ double row_below1(double v) {
   return __builtin_amdgcn_mov_dpp(v, 0x111, 0xf, 0xf, true);
 }
 
-// The loads of v are waited for here, so that a later wait need not include
-// the stores issued in between.
-__device__ __forceinline__ void landed(double& v) { asm volatile("" : "+v"(v)); }
-
 // LDS exchange between lanes of one wavefront: its LDS operations complete
 // in order; the fence keeps the compiler from moving them across.
 __device__ __forceinline__ void wave_sync() {

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/canoe_gpu.h"
+#include "fused64.hpp"
 #include "launch.hpp"
 #include "sphere.hpp"
 #include "sphere_geom.hpp"
@@ -88,8 +89,8 @@ struct cg_run {
   double* h_dt = nullptr;
   double* dt_part = nullptr;  // per-workgroup minima, dt_parts per block
   int dt_parts = 1;
-  // tiles of the fused face kernel over every 3D block (FP32-flux form,
-  // face variants 3 / 4), built for (tile_variant, tile_seg)
+  // tiles of the fused face kernel over every 3D block, built for
+  // (tile_variant, tile_seg)
   KTile* d_tiles = nullptr;
   int ntiles = 0, tile_variant = -1, tile_seg = -1;
   unsigned bc2_grid = 1, bc3_grid = 1;  // workgroups per block of the ghost kernels
@@ -114,10 +115,43 @@ void free_block(RunBlock& b) {
   b = RunBlock();
 }
 
-// Face variants 3 / 4 of the FP32-flux form: one tile launch per stage.
+// 3D blocks whose faces and divergence come from one tile launch per stage:
+// face variants 3 / 4 of the FP32-flux form, and the FP64 form of dry runs
+// (256 x 256 x 128: 1.22 ms per stage against 1.57 for the per-face kernels
+// and the divergence).  With three species the FP64 tile needs 59 KB and one
+// wavefront per SIMD: 75 x 130 x 97 cells 0.47 ms against 0.32 for the
+// per-face kernels, which stay.
 bool fused_tiles(const cg_run* r) {
-  return r->cfg.precision == CG_PREC_FP32 &&
-         (r->tune.face_variant == 3 || r->tune.face_variant == 4);
+  if (r->sph) return false;
+  if (r->cfg.precision == CG_PREC_FP64) return r->N == 5;
+  return r->tune.face_variant == 3 || r->tune.face_variant == 4;
+}
+
+// Columns of a tile.
+constexpr int F64_TJ = 32, F64_TK = 8;
+void tile_shape(const cg_run* r, int& tj, int& tk) {
+  const bool wide = r->cfg.precision == CG_PREC_FP64 || r->tune.face_variant == 3;
+  tj = wide ? 32 : 16;
+  tk = wide ? 8 : 16;
+}
+
+void launch_fused64(cg_run* r, const KSource& src, KTimer* tm) {
+  hipStream_t s = r->ctx->stream;
+  const bool w5h = r->cfg.order_h == 5, w5v = r->cfg.order_v == 5;
+#define CG_FUSED64(OH, OV)                                                           \
+  TIMED(tm, KID_DIVERGENCE,                                                          \
+        (k_fused64_batch<0, OH, OV, F64_TJ, F64_TK>                                  \
+             <<<(unsigned)r->ntiles, F64_TJ * F64_TK, 0, s>>>(r->d_bp, r->d_tiles, r->kt, \
+                                                              src, r->cfg.rsolver)))
+  if (w5h && w5v)
+    CG_FUSED64(5, 5);
+  else if (w5h)
+    CG_FUSED64(5, 2);
+  else if (w5v)
+    CG_FUSED64(2, 5);
+  else
+    CG_FUSED64(2, 2);
+#undef CG_FUSED64
 }
 
 unsigned implicit_grid(const cg_run* r) {
@@ -236,14 +270,14 @@ int run_stage(cg_run* r, int s) {
     const KGrid& g = b.g;
     const long long ncell = (long long)g.nx1 * g.nx2 * g.nx3;
     // implicit runs get psf / psv from the previous downward sweep
-    if (r->cfg.precision == CG_PREC_FP32) {
-      if (tiled && g.f2 && g.f3) {  // faces in the batched tile launch below
-        if (!imp && g.grav != 0.0)
-          TIMED(tm, KID_SCAN,
-                (k_hydrostatic_scan<NM><<<nblk((long long)g.nx2 * g.nx3, 256), 256, 0, st>>>(
+    if (tiled && g.f2 && g.f3) {  // faces in the batched tile launch below
+      if (!imp && g.grav != 0.0)
+        TIMED(tm, KID_SCAN,
+              (k_hydrostatic_scan<NM><<<nblk((long long)g.nx2 * g.nx3, 256), 256, 0, st>>>(
                     g, r->kt, b.w, b.psf, b.psv)));
-        continue;
-      }
+      continue;
+    }
+    if (r->cfg.precision == CG_PREC_FP32) {
       launch_fluxes32<NM>(g, r->kt, r->cfg, src, b.w, b.ff, b.psf, b.psv, b.pref,
                           b.du, st, tm, !imp, bs, r->tune.face_variant,
                           r->tune.march_seg);
@@ -256,7 +290,9 @@ int run_stage(cg_run* r, int s) {
                 g.grav != 0.0 ? b.psv : nullptr, b.du)));
     }
   }
-  if (tiled)
+  if (tiled && r->cfg.precision == CG_PREC_FP64)
+    launch_fused64(r, src, tm);
+  else if (tiled)
     launch_fused_batch<NM>(r->d_bp, r->d_tiles, r->ntiles, r->kt, r->cfg, src,
                            r->tune.face_variant, st, tm);
   // SolveImplicit3D's x3 then x2 lines (solve_implicit_3d.cpp:25-88), with
@@ -608,9 +644,22 @@ int capture(cg_run* r) {
 // capturing).  Tiles of the tallest blocks come first.
 int ensure_tiles(cg_run* r) {
   if (!fused_tiles(r)) return CG_OK;
-  const int v = r->tune.face_variant, seg = r->tune.march_seg;
+  int tj, tk;
+  tile_shape(r, tj, tk);
+  // A segment is at most march_seg levels, and short enough that the tiles
+  // fill the chip four times over (a segment's first x1 face is its only
+  // extra work).
+  long long per_level = 0;
+  for (const RunBlock& rb : r->blocks) {
+    const KGrid& g = rb.g;
+    if (!(g.f2 && g.f3)) continue;
+    const long long nt = ((g.nx2 + tj - 1) / tj) * (long long)((g.nx3 + tk - 1) / tk);
+    per_level += nt * g.nx1;
+  }
+  const long long want = 4LL * r->ncu;
+  const int seg = (int)std::max(1LL, std::min<long long>(r->tune.march_seg, per_level / want));
+  const int v = r->tune.face_variant;
   if (r->d_tiles && r->tile_variant == v && r->tile_seg == seg) return CG_OK;
-  const int tj = (v == 3) ? 32 : 16, tk = (v == 3) ? 8 : 16;
   std::vector<int> order(r->blocks.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
