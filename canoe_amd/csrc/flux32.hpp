@@ -998,7 +998,7 @@ void launch_fluxes32(const KGrid& g, const KThermo& th, const cg_config& cfg,
   float* f3 = f2 + (size_t)(5 + NM) * g.f[1].n;
   if (decomp && scan)
     TIMED(tm, KID_SCAN,
-          (k_hydrostatic_scan<NM><<<(unsigned)((ncol + 255) / 256), 256, 0, s>>>(g, th, w, psf, psv)));
+          (launch_scan<NM>(g, th, w, psf, psv, s)));
   if (variant == 0) {
     const unsigned b1 = (unsigned)((ncol * (g.nx1 + 1) + bs - 1) / bs);
     if (w5v)

@@ -130,6 +130,97 @@ __global__ void __launch_bounds__(256)
   scan_column<NM>(g, th, w, psf, psv, t);
 }
 
+// The same with C columns per workgroup of 256 lanes: the densities of every
+// level are read at once into LDS as steps grav rho dx, C lanes run the
+// recurrences from LDS (downward from the top face, and up through the top
+// ghosts), and all lanes form the logarithmic means.  One column per lane
+// leaves the chip to ncol / 64 wavefronts, each waiting for memory and one
+// logarithm per level; in the AthenaArray layout it also reads a cache line
+// per lane and level.  The steps' products and the order of the sums are the
+// same, so psf and psv are too.
+template <int NM, int C>
+__global__ void __launch_bounds__(256)
+    k_hydrostatic_scan_lds(KGrid g, KThermo th, const double* __restrict__ w,
+                           double* __restrict__ psf, double* __restrict__ psv) {
+  constexpr int IPR = 4 + NM;
+  extern __shared__ double lds[];
+  const long long ncol = (long long)g.nx2 * g.nx3;
+  const long long t0 = (long long)blockIdx.x * C;
+  const int nc = (int)min((long long)C, ncol - t0);
+  double* step = lds;              // [level][C]
+  double* pf = lds + g.nc1 * C;    // [face][C]
+  const int is = g.is, ie = g.ie;
+  const double grav = g.grav, dx = g.dx1;
+  const double gb = (g.bc[0] == 0) ? -grav : grav, gt = (g.bc[1] == 0) ? -grav : grav;
+  const int tid = threadIdx.x;
+  auto item = [&](int e, int n1, int& c, int& i) {  // lanes along the unit stride
+    if (g.lvl) {
+      c = e % C;
+      i = e / C;
+    } else {
+      i = e % n1;
+      c = e / n1;
+    }
+  };
+  for (int e = tid; e < g.nc1 * C; e += 256) {
+    int c, i;
+    item(e, g.nc1, c, i);
+    if (c >= nc) continue;
+    const int j = g.js + (int)((t0 + c) % g.nx2), k = g.ks + (int)((t0 + c) / g.nx2);
+    const double rho = w[g.at(0, k, j, i)];
+    step[i * C + c] = (i < is ? gb : i > ie ? gt : grav) * rho * dx;
+    if (i == ie) {
+      const double p = w[g.at(IPR, k, j, ie)];
+      const double RdTv = p / rho;
+      pf[(ie + 1) * C + c] = p * exp_d(grav * dx / (2 * RdTv));
+    }
+  }
+  __syncthreads();
+  if (tid < nc) {
+    double cur = pf[(ie + 1) * C + tid];
+#pragma unroll 8
+    for (int i = ie; i >= 0; --i) {
+      cur = cur - step[i * C + tid];
+      pf[i * C + tid] = cur;
+    }
+  } else if (tid >= 64 && tid < 64 + nc) {
+    const int c = tid - 64;
+    double cur = pf[(ie + 1) * C + c];
+    for (int i = ie + 1; i <= ie + NG; ++i) {
+      cur = cur + step[i * C + c];
+      pf[(i + 1) * C + c] = cur;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < (g.nc1 + 1) * C; e += 256) {
+    int c, i;
+    item(e, g.nc1 + 1, c, i);
+    if (c >= nc) continue;
+    const long long o = (t0 + c) * g.ps_c + i * g.ps_i;
+    const double lo = pf[i * C + c];
+    psf[o] = lo;
+    if (i < g.nc1) psv[o] = log_mean(lo, pf[(i + 1) * C + c]);
+  }
+}
+
+// psf and psv of every column of a block: 16 columns per workgroup while
+// their two LDS arrays fit 64 KB (255 cells with ghosts), 4 up to 1,023 cells,
+// one column per lane above.
+template <int NM>
+void launch_scan(const KGrid& g, const KThermo& th, const double* w, double* psf, double* psv,
+                 hipStream_t s) {
+  const long long ncol = (long long)g.nx2 * g.nx3;
+  const size_t per = sizeof(double) * (2 * (size_t)g.nc1 + 1);
+  if (per * 16 <= 65536)
+    k_hydrostatic_scan_lds<NM, 16>
+        <<<(unsigned)((ncol + 15) / 16), 256, per * 16, s>>>(g, th, w, psf, psv);
+  else if (per * 4 <= 65536)
+    k_hydrostatic_scan_lds<NM, 4>
+        <<<(unsigned)((ncol + 3) / 4), 256, per * 4, s>>>(g, th, w, psf, psv);
+  else
+    k_hydrostatic_scan<NM><<<(unsigned)((ncol + 255) / 256), 256, 0, s>>>(g, th, w, psf, psv);
+}
+
 // ---------------------------------------------------------------------------
 // K1a: x1 face fluxes with the hydrostatic decomposition around the
 // reconstruction (patches/19.calculate_fluxes.patch:23-47;

@@ -121,7 +121,7 @@ void launch_fluxes(const KGrid& g, const KThermo& th, const cg_config& cfg,
   const int decomp = g.grav != 0.0;
   if (decomp && scan)
     TIMED(tm, KID_SCAN,
-          (k_hydrostatic_scan<NM><<<(unsigned)((ncol + 255) / 256), 256, 0, s>>>(g, th, w, psf, psv)));
+          (launch_scan<NM>(g, th, w, psf, psv, s)));
   const long long n1 = ncol * (g.nx1 + 1);
   if (cfg.order_v == 5)
     TIMED(tm, KID_FLUX_X1,

@@ -273,8 +273,7 @@ int run_stage(cg_run* r, int s) {
     if (tiled && g.f2 && g.f3) {  // faces in the batched tile launch below
       if (!imp && g.grav != 0.0)
         TIMED(tm, KID_SCAN,
-              (k_hydrostatic_scan<NM><<<nblk((long long)g.nx2 * g.nx3, 256), 256, 0, st>>>(
-                    g, r->kt, b.w, b.psf, b.psv)));
+              (launch_scan<NM>(g, r->kt, b.w, b.psf, b.psv, st)));
       continue;
     }
     if (r->cfg.precision == CG_PREC_FP32) {
@@ -349,8 +348,7 @@ int run_stage(cg_run* r, int s) {
               (k_bc_x1<NM><<<nblk((long long)g.nx2 * g.nx3 * NG, 256), 256, 0, st>>>(g, b.w)));
         if (g.grav != 0.0)
           TIMED(tm, KID_SCAN,
-                (k_hydrostatic_scan<NM><<<nblk((long long)g.nx2 * g.nx3, 256), 256, 0, st>>>(
-                    g, r->kt, b.w, b.psf, b.psv)));
+                (launch_scan<NM>(g, r->kt, b.w, b.psf, b.psv, st)));
       }
     }
     // x2 then x3 ghosts of every block (x3 copies the x2 ghosts' corners)
@@ -614,7 +612,7 @@ void prime_block(cg_run* r, RunBlock& b) {
   launch_bc<NM>(g, b.w, s);
   if (b.pref) k_level_mean_p<NM><<<g.nc1, 256, 0, s>>>(g, b.w, b.pref);
   if (g.grav != 0.0)
-    k_hydrostatic_scan<NM><<<nblk(ncol, 256), 256, 0, s>>>(g, r->kt, b.w, b.psf, b.psv);
+    launch_scan<NM>(g, r->kt, b.w, b.psf, b.psv, s);
 }
 
 int ensure_tiles(cg_run* r);
