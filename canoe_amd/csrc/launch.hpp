@@ -196,6 +196,13 @@ inline KLines make_lines(const KGrid& g, int dir) {
 // 0.74, 25,600 columns 1.17 against 0.84; 3 x 3: 9,216 columns 0.29 against
 // 0.40, 16,384 columns 0.42 against 0.41): two rounds.
 constexpr long long ROWS_MAX_LINES = 16384;
+// Periodic lines: about 4.4 us per level and round of 8,192 lines (5 x 5)
+// against 17 to 22 us per level for any number up to 32,768 in the one-lane
+// kernel, whose 65,536 lines would take no longer.  x2 lines of 64 x 128 x
+// 128 cells 0.63 against 2.18 ms, of 128 x 256 x 256 4.51 against 5.55 ms;
+// 3 x 3 x2 lines of 64 x 256 x 128 0.57 against 1.16, x3 lines 0.48 against
+// 0.66 ms.
+constexpr long long rows_max_periodic(int B) { return B == 5 ? 32768 : 16384; }
 
 inline unsigned rows_grid(long long nline) { return nblk(nline, RLINES * RWAVES); }
 
@@ -253,6 +260,10 @@ void launch_lines_d(const KLines& L, const KThermo& th, double dt, const double*
     TIMED(tm, KID_LINES,
           (k_rows_walls<NM, B, DIR><<<rows_grid(L.nline), 64 * RWAVES, 0, s>>>(
               L, th, dt, dtp, true, true, w, du, lv, status)));
+  else if (per && L.nline <= rows_max_periodic(B))
+    TIMED(tm, KID_LINES,
+          (k_rows_periodic<NM, B, DIR><<<rows_grid(L.nline), 64 * RWAVES, 0, s>>>(
+              L, th, dt, dtp, w, du, lv, status)));
   else if (per)
     TIMED(tm, KID_LINES,
           (k_line_periodic<NM, B, DIR><<<nb, 64, 0, s>>>(L, th, dt, dtp, w, du, lv, status)));

@@ -217,10 +217,10 @@ struct RowAsm {
     }
   }
   // records of the fetched chunk; fold_lo, fold_hi: reflecting walls at the
-  // line's ends.  next_b (periodic lines): b of the level above the lane's.
+  // line's ends; seven: the next chunk starts at the eighth lane's level
   __device__ __forceinline__ void store(int i, bool fold_lo, bool fold_hi,
                                         double* __restrict__ cols, double* __restrict__ bm,
-                                        Mt<B>* next_b) {
+                                        bool seven = false) {
     constexpr int NC = RowRec<B>::NC;
     i = min(i, hi);
     if (out_lo && i == L.lo)
@@ -236,7 +236,7 @@ struct RowAsm {
       for (int q = 0; q < B; ++q) {
         const double v = row_below1(Ap.a[r][q]);
         Am.a[r][q] = first ? below.a[r][q] : v;
-        below.a[r][q] = oct_bcast<OCT - 1>(Ap.a[r][q]);
+        below.a[r][q] = seven ? oct_bcast<OCT - 2>(Ap.a[r][q]) : oct_bcast<OCT - 1>(Ap.a[r][q]);
       }
     jac(wm, dm);
     jac(wp, dp);
@@ -254,14 +254,6 @@ struct RowAsm {
         b.a[r][q] = -(Am.a[r][q] + dm.a[r][q]) * L.sla;
         c.a[r][q] = -(Ap.a[r][q] - dp.a[r][q]) * L.sra;
       }
-    if (next_b) {
-      Mt<B> dc;
-      jac(wc, dc);
-#pragma unroll
-      for (int r = 0; r < B; ++r)
-#pragma unroll
-        for (int q = 0; q < B; ++q) next_b->a[r][q] = -(Ap.a[r][q] + dc.a[r][q]) * L.sla;
-    }
     if (fold_lo && i == L.lo) {
 #pragma unroll
       for (int r = 0; r < B; ++r)
@@ -370,7 +362,7 @@ __device__ __forceinline__ bool oct_forward(RowAsm<NM, B, DIR>& as, double* __re
   as.fetch(lo + l8);
   as.land();
   for (int p0 = 0; p0 < n; p0 += OCT) {
-    as.store(lo + p0 + l8, fold_lo, fold_hi, cols + lane * COLS, bms + lane * BM, nullptr);
+    as.store(lo + p0 + l8, fold_lo, fold_hi, cols + lane * COLS, bms + lane * BM);
     wave_sync();
     if (p0 + OCT < n) as.fetch(lo + p0 + OCT + l8);
     const int m = min(OCT, n - p0);
@@ -401,6 +393,22 @@ __device__ __forceinline__ bool oct_forward(RowAsm<NM, B, DIR>& as, double* __re
   return ok;
 }
 
+// a . x of a row a with the vector whose component k lane k of the octet
+// holds, terms in order.
+template <int B>
+struct OctDot {
+  template <int K>
+  static __device__ __forceinline__ double term(const double* a, double x) {
+    if constexpr (K == 0)
+      return a[0] * oct_bcast<0>(x);
+    else
+      return term<K - 1>(a, x) + a[K] * oct_bcast<K>(x);
+  }
+  static __device__ __forceinline__ double dot(const double* a, double x) {
+    return term<B - 1>(a, x);
+  }
+};
+
 // Back substitution of a chunk of eight levels from p0, top down: the
 // records pass from one per lane through LDS to one row per lane; lane r of
 // the octet carries component r of the solution x (that of the level above,
@@ -419,13 +427,6 @@ struct OctBack {
     const double2* a = ar.at(max(p0, 0), lane / OCT, lane & (OCT - 1), step);
 #pragma unroll
     for (int k = 0; k < A::PAIRS; ++k) buf[k] = a[(long long)k * step];
-  }
-  template <int K>
-  __device__ __forceinline__ double dot(const double* a) const {
-    if constexpr (K == 0)
-      return a[0] * oct_bcast<0>(x);
-    else
-      return dot<K - 1>(a) + a[K] * oct_bcast<K>(x);
   }
   // sa: 64 LS doubles for the records, sd: 64 B doubles for the solution
   __device__ __forceinline__ void land() {
@@ -457,7 +458,7 @@ struct OctBack {
 #pragma unroll
     for (int h = OCT - 1; h >= 0; --h) {
       if (p0 + h >= ar.n) continue;
-      const double s = dot<B - 1>(v[h]);
+      const double s = OctDot<B>::dot(v[h], x);
       x = (p0 + h == ar.n - 1) ? v[h][B] : v[h][B] - s;
       if (l8 < B) px[h * B] = x;
     }
@@ -518,6 +519,273 @@ __global__ void __launch_bounds__(64 * RWAVES)
     cell.land();
     if (p < L.n && line < nl)
       line_store<NM, B, DIR, false>(d, c, du, o + (long long)(L.lo + p) * L.sl, L.sn);
+  }
+}
+
+// A periodic line (k_line_periodic, lines.hpp, whose recurrences and order of
+// operations these are) with eight lanes: lane q < B holds column q of ainv, U
+// (= c), gamma and of the products, lane B the vector zeta in gamma's place.
+// Left factors pass through LDS: T = b ainv_{p-1} and beta U are written by
+// columns and read whole by every lane.  A level's record is free once its
+// columns are in registers; the products use its slots, and at the end of the
+// level it holds what the way back needs, row r as [zeta | U | gamma] (B (2B
+// + 1) doubles) and ainv (B B): 80 doubles per cell instead of the one-lane
+// kernel's 105.
+template <int B>
+__device__ __forceinline__ void mat_col(const double* x, const double* y, double* z) {
+#pragma unroll
+  for (int r = 0; r < B; ++r) {
+    double s = x[r * B] * y[0];
+#pragma unroll
+    for (int k = 1; k < B; ++k) s += x[r * B + k] * y[k];
+    z[r] = s;
+  }
+}
+
+template <int NM, int B, int DIR>
+__global__ void __launch_bounds__(64 * RWAVES)
+    k_rows_periodic(KLines L, KThermo th, double dt, const double* __restrict__ dtp,
+                    const double* __restrict__ w, double* __restrict__ du,
+                    double* __restrict__ lv, int* __restrict__ status) {
+  constexpr int NC = RowRec<B>::NC, COLS = RowRec<B>::COLS, BM = RowRec<B>::BM;
+  constexpr int PAIRS = (COLS + BM) / 2;
+  static_assert(2 * PAIRS == COLS + BM, "records go out in pairs");
+  __shared__ double shm[RWAVES * RowRec<B>::WAVE];
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const long long line0 = ((long long)blockIdx.x * RWAVES + wv) * RLINES;
+  if (line0 >= L.nline) return;  // whole wavefronts; no workgroup barrier below
+  double* cols = shm + wv * RowRec<B>::WAVE;
+  double* bms = cols + 64 * COLS;
+  const int lane = threadIdx.x & 63, line = lane / OCT, l8 = lane & (OCT - 1);
+  const int nl = (int)min((long long)RLINES, L.nline - line0);
+  const long long t = line0 + min(line, nl - 1);
+  const long long o = L.org(t);
+  const int n = L.n, lo = L.lo;
+  double2* ar = reinterpret_cast<double2*>(lv + line0 * n * (COLS + BM));
+  if (dtp) dt = dt * dtp[0];
+  RowAsm<NM, B, DIR> as(L, th, w, du, o, dt, nullptr, 0, false, false);
+  // chunks of eight levels; the first has seven where the last level would
+  // otherwise start a chunk, since level n - 2 reads level n - 1's b
+  const int first = ((n - 1) % OCT == 0) ? OCT - 1 : OCT;
+  const int q = l8 < B ? l8 : 0;
+  const bool is_z = l8 == B, is_c = l8 < B;
+  bool ok = true;
+  double bf[BM];              // beta_{p-1}, whole (at first the corner c_{lo-1})
+  double ai[B], U[B], gm[B];  // the lane's columns of level p - 1
+  double sb[B];               // sum of beta gamma (lane B: beta zeta)
+  {
+    Mt<B> um1;
+    as.start(&um1);
+#pragma unroll
+    for (int r = 0; r < B; ++r) {
+      sb[r] = 0.0;
+      ai[r] = U[r] = gm[r] = 0.0;
+#pragma unroll
+      for (int k = 0; k < B; ++k) bf[r * B + k] = um1.a[r][k];
+    }
+  }
+  as.fetch(lo + l8);
+  as.land();
+  auto flush = [&](int p0, int m) {
+    if (l8 < m && line < nl) {
+      const double* c = cols + lane * COLS;
+      const double* b = bms + lane * BM;
+      double2* dst = ar + (long long)p0 * PAIRS * nl + line * m + l8;
+#pragma unroll
+      for (int k = 0; k < PAIRS; ++k) {
+        const int e0 = 2 * k, e1 = 2 * k + 1;
+        dst[(long long)k * nl * m] = double2{e0 < COLS ? c[e0] : b[e0 - COLS],
+                                             e1 < COLS ? c[e1] : b[e1 - COLS]};
+      }
+    }
+  };
+  double xl = 0.0;  // component min(l8, B - 1) of the last level's solution
+  for (int p0 = 0, len = first; p0 < n; p0 += len, len = OCT) {
+    as.store(lo + p0 + l8, false, false, cols + lane * COLS, bms + lane * BM, len < OCT);
+    wave_sync();
+    if (p0 + len < n) as.fetch(lo + p0 + len + l8);
+    const int m = min(len, n - p0);
+    for (int l = 0; l < m; ++l) {
+      const int p = p0 + l;
+      double* rc = cols + (lane - l8 + l) * COLS;
+      double* rb = bms + (lane - l8 + l) * BM;
+      double a[B], c[B], tmp[BM];
+#pragma unroll
+      for (int r = 0; r < B; ++r) {
+        a[r] = rc[r * NC + (is_z ? 2 * B : q)];  // lane B: the right-hand side
+        c[r] = rc[r * NC + B + q];
+      }
+      double x[B], inv[B];
+      if (p == n - 1) {
+        // ainv = (a - sum beta gamma)^-1, zeta = r - sum beta zeta
+#pragma unroll
+        for (int r = 0; r < B; ++r) {
+          a[r] = a[r] - sb[r];
+          inv[r] = (r == q) ? 1.0 : 0.0;
+        }
+        wave_sync();
+        if (is_z) {
+#pragma unroll
+          for (int r = 0; r < B; ++r) rc[r] = a[r];
+        }
+        gj_oct<B, false>(a, inv, ok);
+        if (is_c) {
+#pragma unroll
+          for (int r = 0; r < B; ++r) rb[r * B + q] = inv[r];
+        }
+        wave_sync();
+        const int rr = min(l8, B - 1);
+        double s = rb[rr * B] * rc[0];
+#pragma unroll
+        for (int k = 1; k < B; ++k) s += rb[rr * B + k] * rc[k];
+        xl = s;
+        wave_sync();
+        break;
+      }
+#pragma unroll
+      for (int e = 0; e < BM; ++e) tmp[e] = rb[e];
+      double gnew[B], bu[B];
+      if (p == 0) {
+        // gamma_0 = b_0, zeta_0 = r_0
+#pragma unroll
+        for (int r = 0; r < B; ++r) gnew[r] = is_z ? a[r] : rb[r * B + q];
+      } else {
+        double T[B];
+        mat_col<B>(tmp, ai, T);  // T = b ainv_{p-1}
+        wave_sync();
+        if (is_c) {
+#pragma unroll
+          for (int r = 0; r < B; ++r) rb[r * B + q] = T[r];
+        }
+        wave_sync();
+#pragma unroll
+        for (int e = 0; e < BM; ++e) tmp[e] = rb[e];
+        mat_col<B>(tmp, gm, x);  // T gamma_{p-1}, lane B: T zeta_{p-1}
+#pragma unroll
+        for (int r = 0; r < B; ++r)
+          gnew[r] = is_z ? a[r] - x[r] : p < n - 2 ? -x[r] : c[r] - x[r];
+        mat_col<B>(tmp, U, x);
+#pragma unroll
+        for (int r = 0; r < B; ++r) a[r] = a[r] - x[r];
+        mat_col<B>(bf, U, bu);  // beta_{p-1} U_{p-1}
+        if (p == n - 2) {       // L_{n-1} - beta_{n-3} U_{n-3}
+#pragma unroll
+          for (int r = 0; r < B; ++r) bu[r] = rb[BM + r * B + q] - bu[r];
+        }
+        wave_sync();
+        if (is_c) {
+#pragma unroll
+          for (int r = 0; r < B; ++r) rc[r * B + q] = bu[r];
+        }
+        wave_sync();
+#pragma unroll
+        for (int e = 0; e < BM; ++e) bf[e] = rc[e];
+      }
+#pragma unroll
+      for (int r = 0; r < B; ++r) inv[r] = (r == q) ? 1.0 : 0.0;
+      gj_oct<B, false>(a, inv, ok);
+      mat_col<B>(bf, inv, bu);  // beta_p
+      if (p > 0 && p < n - 2) {
+#pragma unroll
+        for (int r = 0; r < B; ++r) bu[r] = -bu[r];
+      }
+      wave_sync();
+      if (is_c) {
+#pragma unroll
+        for (int r = 0; r < B; ++r) rc[r * B + q] = bu[r];
+      }
+      wave_sync();
+#pragma unroll
+      for (int e = 0; e < BM; ++e) bf[e] = rc[e];
+      mat_col<B>(bf, gnew, x);
+#pragma unroll
+      for (int r = 0; r < B; ++r) {
+        sb[r] = sb[r] + x[r];
+        ai[r] = inv[r];
+        U[r] = c[r];
+        gm[r] = gnew[r];
+      }
+      wave_sync();
+      if (l8 <= B) {
+#pragma unroll
+        for (int r = 0; r < B; ++r) {
+          rc[r * NC + (is_z ? 0 : 1 + B + q)] = gnew[r];
+          if (is_c) {
+            rc[r * NC + 1 + q] = c[r];
+            rb[r * B + q] = inv[r];
+          }
+        }
+      }
+    }
+    as.land();
+    wave_sync();
+    flush(p0, m);
+    wave_sync();
+  }
+  if (!ok && line < nl) atomicOr(status, 1);
+  archive_fence();
+  // the way back, top chunk first: lane r holds component r of x
+  double2 buf[PAIRS];
+  LineCell<NM, DIR> cell;
+  auto length = [&](int p0) { return p0 == 0 ? min(first, n) : min(OCT, n - p0); };
+  auto fetch = [&](int p0) {
+    const int m = length(p0);
+    const double2* src = ar + (long long)p0 * PAIRS * nl + min(line, nl - 1) * m + min(l8, m - 1);
+#pragma unroll
+    for (int k = 0; k < PAIRS; ++k) buf[k] = src[(long long)k * nl * m];
+    cell.load(L, w, du, o, t, lo + p0 + min(l8, m - 1), false);
+  };
+  auto land = [&]() {
+#pragma unroll
+    for (int k = 0; k < PAIRS; ++k) {
+      landed(buf[k].x);
+      landed(buf[k].y);
+    }
+    cell.land();
+  };
+  const int rr = min(l8, B - 1);
+  double xv = xl;
+  int p0 = n <= first ? 0 : first + (n - 1 - first) / OCT * OCT;
+  fetch(p0);
+  land();
+  while (true) {
+    const int m = length(p0);
+    wave_sync();
+    {
+      double* c = cols + lane * COLS;
+      double* b = bms + lane * BM;
+#pragma unroll
+      for (int k = 0; k < PAIRS; ++k) {
+        const int e0 = 2 * k, e1 = 2 * k + 1;
+        (e0 < COLS ? c[e0] : b[e0 - COLS]) = buf[k].x;
+        (e1 < COLS ? c[e1] : b[e1 - COLS]) = buf[k].y;
+      }
+    }
+    const LineCell<NM, DIR> mine = cell;
+    const int next = p0 == 0 ? -1 : p0 == first ? 0 : p0 - OCT;
+    if (next >= 0) fetch(next);
+    wave_sync();
+    for (int l = m - 1; l >= 0; --l) {
+      double* rc = cols + (lane - l8 + l) * COLS + rr * NC;
+      const double* rb = bms + (lane - l8 + l) * BM + rr * B;
+      if (p0 + l < n - 1) {
+        double ux = 0.0;
+        if (p0 + l < n - 2) ux = OctDot<B>::dot(rc + 1, xv);
+        const double gx = OctDot<B>::dot(rc + 1 + B, xl);
+        const double tv = (rc[0] - ux) - gx;
+        xv = OctDot<B>::dot(rb, tv);
+      }
+      if (l8 < B) rc[0] = xv;
+    }
+    wave_sync();
+    Vt<B> d;
+#pragma unroll
+    for (int r = 0; r < B; ++r) d.v[r] = cols[lane * COLS + r * NC];
+    land();
+    if (l8 < m && line < nl)
+      line_store<NM, B, DIR, true>(d, mine, du, o + (long long)(lo + p0 + l8) * L.sl, L.sn);
+    if (next < 0) break;
+    p0 = next;
   }
 }
 

@@ -84,3 +84,19 @@ def test_run_stage_equals_the_one_lane_kernels(ctx, config, flag, dims, bc1):
     for a, b in zip(*out):
         assert np.all(np.isfinite(a[:, blk.interior()[0], blk.interior()[1]]))
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("flag", [2, 4, 10, 12, 15, 7])
+@pytest.mark.parametrize("dims", [(3, 3, 3), (5, 8, 9), (4, 9, 17), (3, 16, 10),
+                                  (6, 25, 7), (9, 5, 11)])
+def test_caller_periodic_lines_equal_the_oracle(ctx, flag, dims):
+    """Periodic x2 / x3 lines whose last level falls on every place of a chunk
+    of eight (lines of 9, 17 and 25 cells start with a chunk of seven)."""
+    blk, th, cfg, w = perturbed_state(2, dims)
+    du = _increments(blk, 7)
+    print("periodic flag=%d dims=%s" % (flag, dims), flush=True)
+    got = ca.ImplicitSolver(ctx, blk, th, flag).solve_implicit_3d(du, w, 0.4)
+    ref, r = orl.implicit_solve(blk, th, du, w, 0.4, flag)
+    assert r == 0
+    sk, sj, si = blk.interior()
+    assert relerr(got[:, sk, sj, si], ref[:, sk, sj, si]) <= TOL
