@@ -56,10 +56,8 @@ template <> struct Lay<3> { enum { IN = 64, OUT = 3, W = 8640, B = 8832, H = 132
 constexpr int HROWS = 196, DZROWS = 195;
 
 // ---------------------------------------------------------------------------
-// Elementwise routines: the same algorithms as the oracle (bf16 round to
-// nearest even; Cody-Waite exp with the 0.693359375 - 2.12194440e-4 split of
-// ln2 and a Taylor series through r^6; tanh-form GELU), single precision,
-// no contraction.
+// Elementwise routines in single precision, no contraction: bf16 round to
+// nearest even, tanh-form GELU.
 CG_HD uint16_t bf16_bits(float f) {
   uint32_t u = __builtin_bit_cast(uint32_t, f);
   if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
@@ -71,38 +69,30 @@ CG_HD float bf16_float(uint16_t h) {
   return __builtin_bit_cast(float, (uint32_t)h << 16);
 }
 
-CG_HD float exp_f(float x) {
-  if (x != x) return x;
-  if (x > 88.0f) return __builtin_huge_valf();
-  if (x < -87.0f) return 0.0f;
-  float kf = floorf(x * 1.44269504f + 0.5f);
-  float r = (x - kf * 0.693359375f) - kf * -2.12194440e-4f;
-  float p = 1.38888889e-3f;
-  p = p * r + 8.33333333e-3f;
-  p = p * r + 4.16666667e-2f;
-  p = p * r + 1.66666667e-1f;
-  p = p * r + 0.5f;
-  p = p * r + 1.0f;
-  p = p * r + 1.0f;
-  return ldexpf(p, (int)kf);
+// tanh-form GELU (Hendrycks & Gimpel 2016) by its sigmoid: with e = e^(2u), r =
+// 1 / (e + 1) and s = e r (1 - r above zero), (1 + tanh u) / 2 = s and 1 - tanh^2 u = 4 s r,
+// without the differences that lose digits at either end.  The hardware's
+// exponential (of 2 to the power, 1 / ln 2 folded into the factor of u) and
+// reciprocal take a dozen instructions instead of about 50 for a polynomial
+// exponential with a correctly rounded division, which were four fifths of
+// the forward pass.  The exponent is capped so that e stays finite.
+struct Sig {
+  float s, r;
+};
+__device__ __forceinline__ Sig gelu_sig(float z) {
+  const float z3 = (z * z) * z;
+  const float u2 = 2.30220820f * (z + 0.044715f * z3);  // 2 sqrt(2 / pi) / ln 2
+  const float e = __builtin_amdgcn_exp2f(fminf(u2, 126.0f));
+  const float r = __builtin_amdgcn_rcpf(e + 1.0f);
+  return Sig{z > 0.0f ? 1.0f - r : e * r, r};
 }
 
-CG_HD float gelu_tanh(float z) {
-  float z3 = (z * z) * z;
-  float u = 0.797884583f * (z + 0.044715f * z3);
-  float e = exp_f(2.0f * u);
-  return 1.0f - 2.0f / (e + 1.0f);
-}
+__device__ __forceinline__ float gelu(float z) { return z * gelu_sig(z).s; }
 
-CG_HD float gelu(float z) {
-  float t = gelu_tanh(z);
-  return (0.5f * z) * (1.0f + t);
-}
-
-CG_HD float gelu_grad(float z) {
-  float t = gelu_tanh(z);
-  float dudz = 0.797884583f * (1.0f + 0.134145f * (z * z));
-  return 0.5f * (1.0f + t) + (0.5f * z) * ((1.0f - t * t) * dudz);
+__device__ __forceinline__ float gelu_grad(float z) {
+  const Sig g = gelu_sig(z);
+  const float dudz = 0.797884583f * (1.0f + 0.134145f * (z * z));
+  return g.s + (2.0f * z) * ((g.s * g.r) * dudz);
 }
 
 CG_HD uint32_t pack2(uint16_t lo, uint16_t hi) {
@@ -165,12 +155,16 @@ __device__ __forceinline__ u32x4 ldtile(const uint16_t* __restrict__ tiles, int 
   return *(reinterpret_cast<const u32x4*>(tiles + (size_t)t * TILE) + lane);
 }
 
-// bf16 pairs of 16 D tiles: [feature tile][sample tile][pair]
+// bf16 pairs of 4 S D tiles: [feature tile][sample tile][pair].  A wavefront
+// carries S sample tiles of 16: four where it holds a sample per lane, one
+// where samples are few, so that four times as many wavefronts share them.
+template <int S>
 struct Hid {
-  uint32_t h[4][4][2];
+  uint32_t h[4][S][2];
 };
 
-__device__ __forceinline__ u32x4 bop(const Hid& H, int kk, int s) {
+template <int S>
+__device__ __forceinline__ u32x4 bop(const Hid<S>& H, int kk, int s) {
   return u32x4{H.h[2 * kk][s][0], H.h[2 * kk][s][1], H.h[2 * kk + 1][s][0],
                H.h[2 * kk + 1][s][1]};
 }
@@ -195,23 +189,24 @@ __device__ __forceinline__ void input_bop(const float xin[4], u32x4 b[4]) {
   }
 }
 
+template <int S>
 __device__ __forceinline__ void layer1(const uint16_t* __restrict__ tiles,
-                              const float* __restrict__ P, const u32x4 b[4],
-                              f32x4 acc[4][4]) {
+                              const float* __restrict__ P, const u32x4 b[S],
+                              f32x4 acc[4][S]) {
   const int lane = threadIdx.x & 63, g = lane >> 4;
 #pragma unroll
   for (int ot = 0; ot < 4; ++ot) {
     u32x4 a = ldtile(tiles, TF1 + ot, lane);
     f32x4 c0 = bias4(P + Lay<0>::B, 16 * ot + 4 * g, 64);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) acc[ot][s] = mfma(a, b[s], c0);
+    for (int s = 0; s < S; ++s) acc[ot][s] = mfma(a, b[s], c0);
   }
 }
 
-template <int TF, int L>
+template <int TF, int L, int S>
 __device__ __forceinline__ void layer64(const uint16_t* __restrict__ tiles,
-                               const float* __restrict__ P, const Hid& H,
-                               f32x4 acc[4][4]) {
+                               const float* __restrict__ P, const Hid<S>& H,
+                               f32x4 acc[4][S]) {
   const int lane = threadIdx.x & 63, g = lane >> 4;
 #pragma unroll
   for (int ot = 0; ot < 4; ++ot) {
@@ -219,27 +214,29 @@ __device__ __forceinline__ void layer64(const uint16_t* __restrict__ tiles,
     u32x4 a1 = ldtile(tiles, TF + 2 * ot + 1, lane);
     f32x4 c0 = bias4(P + Lay<L>::B, 16 * ot + 4 * g, 64);
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < S; ++s)
       acc[ot][s] = mfma(a1, bop(H, 1, s), mfma(a0, bop(H, 0, s), c0));
   }
 }
 
+template <int S>
 __device__ __forceinline__ void layer_out(const uint16_t* __restrict__ tiles,
-                                 const float* __restrict__ P, const Hid& H,
-                                 f32x4 out[4]) {
+                                 const float* __restrict__ P, const Hid<S>& H,
+                                 f32x4 out[S]) {
   const int lane = threadIdx.x & 63, g = lane >> 4;
   u32x4 a0 = ldtile(tiles, TF4, lane), a1 = ldtile(tiles, TF4 + 1, lane);
   f32x4 c0 = bias4(P + Lay<3>::B, 4 * g, 3);
 #pragma unroll
-  for (int s = 0; s < 4; ++s)
+  for (int s = 0; s < S; ++s)
     out[s] = mfma(a1, bop(H, 1, s), mfma(a0, bop(H, 0, s), c0));
 }
 
-__device__ __forceinline__ void activate(const f32x4 acc[4][4], Hid& H) {
+template <int S>
+__device__ __forceinline__ void activate(const f32x4 acc[4][S], Hid<S>& H) {
 #pragma unroll
   for (int ot = 0; ot < 4; ++ot)
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < S; ++s)
 #pragma unroll
       for (int p = 0; p < 2; ++p)
         H.h[ot][s][p] = pack2(bf16_bits(gelu(acc[ot][s][2 * p])),
@@ -259,22 +256,29 @@ __device__ __forceinline__ void own_output(const f32x4 out[4], float y[3]) {
     }
 }
 
+template <int S>
+__device__ __forceinline__ void forward_tiles(const uint16_t* __restrict__ tiles,
+                                     const float* __restrict__ P,
+                                     const u32x4 b1[S], f32x4 out[S]) {
+  f32x4 acc[4][S];
+  Hid<S> H;
+  layer1<S>(tiles, P, b1, acc);
+  activate<S>(acc, H);
+  layer64<TF2, 1, S>(tiles, P, H, acc);
+  activate<S>(acc, H);
+  layer64<TF3, 2, S>(tiles, P, H, acc);
+  activate<S>(acc, H);
+  layer_out<S>(tiles, P, H, out);
+}
+
 // Forward pass of the wave's 64 samples; xin / y are this lane's sample.
 __device__ __forceinline__ void forward_wave(const uint16_t* __restrict__ tiles,
                                     const float* __restrict__ P,
                                     const float xin[4], float y[3]) {
   u32x4 b1[4];
   input_bop(xin, b1);
-  f32x4 acc[4][4];
-  Hid H;
-  layer1(tiles, P, b1, acc);
-  activate(acc, H);
-  layer64<TF2, 1>(tiles, P, H, acc);
-  activate(acc, H);
-  layer64<TF3, 2>(tiles, P, H, acc);
-  activate(acc, H);
   f32x4 out[4];
-  layer_out(tiles, P, H, out);
+  forward_tiles<4>(tiles, P, b1, out);
   own_output(out, y);
 }
 
@@ -291,6 +295,33 @@ __global__ void __launch_bounds__(256)
   if (valid)
 #pragma unroll
     for (int v = 0; v < 3; ++v) y[c * 3 + v] = yo[v];
+}
+
+// B operand of layer 1 for one tile: lanes 0..15 hold their sample's inputs.
+__device__ __forceinline__ u32x4 input_tile(const float xin[4]) {
+  const bool in = (threadIdx.x & 63) < 16;
+  return in ? u32x4{pack2(bf16_bits(xin[0]), bf16_bits(xin[1])),
+                    pack2(bf16_bits(xin[2]), bf16_bits(xin[3])), 0u, 0u}
+            : u32x4{0u, 0u, 0u, 0u};
+}
+
+// The same with one sample tile per wavefront (few samples).
+__global__ void __launch_bounds__(256)
+    k_mlp_infer_tile(const uint16_t* __restrict__ tiles, const float* __restrict__ P,
+                     long long n, const float* __restrict__ x, float* __restrict__ y) {
+  const int lane = threadIdx.x & 63;
+  const long long c = ((long long)blockIdx.x * 4 + (threadIdx.x >> 6)) * 16 + (lane & 15);
+  const bool valid = c < n && lane < 16;
+  float xin[4] = {0.f, 0.f, 0.f, 0.f};
+  if (valid)
+#pragma unroll
+    for (int f = 0; f < 4; ++f) xin[f] = x[c * 4 + f];
+  const u32x4 b1[1] = {input_tile(xin)};
+  f32x4 out[1];
+  forward_tiles<1>(tiles, P, b1, out);
+  if (valid)
+#pragma unroll
+    for (int v = 0; v < 3; ++v) y[c * 3 + v] = out[0][v];
 }
 
 // ---------------------------------------------------------------------------
@@ -314,217 +345,203 @@ __device__ __forceinline__ long long sample_of(long long pos, long long nb,
   return (long long)(sm64_next(st) % (uint64_t)npairs);
 }
 
-// Forward with saved pre-activations and feature-major layer inputs, then the
-// backward data pass dY -> dZ3 -> dZ2 -> dZ1 (dZ stored feature-major, fp32).
-// grid = nbp / 256 blocks of 256 (4 waves x 64 samples).
+// Forward and backward data pass (dY -> dZ3 -> dZ2 -> dZ1) of one sample tile
+// per wavefront: the pre-activations stay in registers, the layer inputs (bf16)
+// and dZ (fp32) go out feature-major for the weight gradients.  A batch of
+// 8,192 gives 512 wavefronts; with four tiles per wavefront and the
+// pre-activations through memory it gave 128 and took 107 us.
+// grid = nbp / 64 blocks of 256 (4 waves x 16 samples).
 __global__ void __launch_bounds__(256)
     k_mlp_fb(const uint16_t* __restrict__ tiles, const float* __restrict__ P,
              long long nb, long long nbp, long long npairs,
              const float* __restrict__ X, const float* __restrict__ T,
-             uint64_t seed, int random, float scale, float* __restrict__ zbuf,
-             uint16_t* __restrict__ hbuf, float* __restrict__ dzbuf,
-             float* __restrict__ lossp) {
+             uint64_t seed, int random, float scale, uint16_t* __restrict__ hbuf,
+             float* __restrict__ dzbuf, float* __restrict__ lossp) {
   const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
   const long long wave = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const long long base = wave * 64;
-  long long idx = sample_of(base + lane, nb, npairs, seed, random);
+  const long long pos = wave * 16 + r;  // the lane's sample, in every group g
+  const long long idx = sample_of(pos, nb, npairs, seed, random);
   float xin[4] = {0.f, 0.f, 0.f, 0.f};
   if (idx >= 0)
 #pragma unroll
     for (int f = 0; f < 4; ++f) xin[f] = X[idx * 4 + f];
+  if (lane < 16)
 #pragma unroll
-  for (int f = 0; f < 4; ++f) hbuf[f * nbp + base + lane] = bf16_bits(xin[f]);
-  u32x4 b1[4];
-  input_bop(xin, b1);
-  f32x4 acc[4][4];
-  Hid H;
-  float* zw = zbuf + (size_t)wave * 3 * 4096;
-  auto save = [&](int l, int hrow) {
+    for (int f = 0; f < 4; ++f) hbuf[f * nbp + pos] = bf16_bits(xin[f]);
+  const u32x4 b1[1] = {input_tile(xin)};
+  f32x4 z[3][4][1];
+  Hid<1> H;
+  auto save = [&](int hrow) {
 #pragma unroll
     for (int ot = 0; ot < 4; ++ot)
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          zw[(((l * 4 + ot) * 4 + s) * 4 + v) * 64 + lane] = acc[ot][s][v];
-          const int f = 16 * ot + 4 * g + v;
-          const uint32_t hp = H.h[ot][s][v >> 1];
-          hbuf[(hrow + f) * nbp + base + 16 * s + r] =
-              (uint16_t)((v & 1) ? (hp >> 16) : (hp & 0xffffu));
-        }
+      for (int v = 0; v < 4; ++v) {
+        const uint32_t hp = H.h[ot][0][v >> 1];
+        hbuf[(hrow + 16 * ot + 4 * g + v) * nbp + pos] =
+            (uint16_t)((v & 1) ? (hp >> 16) : (hp & 0xffffu));
+      }
   };
-  layer1(tiles, P, b1, acc);
-  activate(acc, H);
-  save(0, Lay<1>::H);
-  layer64<TF2, 1>(tiles, P, H, acc);
-  activate(acc, H);
-  save(1, Lay<2>::H);
-  layer64<TF3, 2>(tiles, P, H, acc);
-  activate(acc, H);
-  save(2, Lay<3>::H);
-  f32x4 out[4];
-  layer_out(tiles, P, H, out);
+  layer1<1>(tiles, P, b1, z[0]);
+  activate<1>(z[0], H);
+  save(Lay<1>::H);
+  layer64<TF2, 1, 1>(tiles, P, H, z[1]);
+  activate<1>(z[1], H);
+  save(Lay<2>::H);
+  layer64<TF3, 2, 1>(tiles, P, H, z[2]);
+  activate<1>(z[2], H);
+  save(Lay<3>::H);
+  f32x4 out[1];
+  layer_out<1>(tiles, P, H, out);
 
   // output gradient dY = (y - t) * 2 / (3 nb)
-  float sse = 0.f;
-  u32x4 dyb[4];
+  float sse = 0.f, d[4];
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    const long long ps = base + 16 * s + r;
-    const long long is = sample_of(ps, nb, npairs, seed, random);
-    float d[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      float dv = 0.f;
-      if (g == 0 && v < 3 && is >= 0) {
-        float e = out[s][v] - T[is * 3 + v];
-        sse += e * e;
-        dv = e * scale;
-      }
-      d[v] = dv;
-      if (g == 0 && v < 3) dzbuf[(Lay<3>::DZ + v) * nbp + ps] = dv;
+  for (int v = 0; v < 4; ++v) {
+    float dv = 0.f;
+    if (g == 0 && v < 3 && idx >= 0) {
+      float e = out[0][v] - T[idx * 3 + v];
+      sse += e * e;
+      dv = e * scale;
     }
-    dyb[s] = u32x4{pack2(bf16_bits(d[0]), bf16_bits(d[1])),
-                   pack2(bf16_bits(d[2]), bf16_bits(d[3])), 0u, 0u};
+    d[v] = dv;
+    if (g == 0 && v < 3) dzbuf[(Lay<3>::DZ + v) * nbp + pos] = dv;
   }
+  const u32x4 dyb = u32x4{pack2(bf16_bits(d[0]), bf16_bits(d[1])),
+                          pack2(bf16_bits(d[2]), bf16_bits(d[3])), 0u, 0u};
   // dH3 = W4^T dY, dZ3 = dH3 gelu'(Z3)
-  f32x4 dh[4][4];
+  f32x4 dh[4];
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int it = 0; it < 4; ++it) {
-    u32x4 a = ldtile(tiles, TB4 + it, lane);
+  for (int it = 0; it < 4; ++it) dh[it] = mfma(ldtile(tiles, TB4 + it, lane), dyb, zero);
+  Hid<1> DZ;
+  auto grad_act = [&](const f32x4 zl[4][1], int dzrow) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) dh[it][s] = mfma(a, dyb[s], zero);
-  }
-  Hid DZ;
-  auto grad_act = [&](int l, int dzrow) {
+    for (int it = 0; it < 4; ++it) {
+      float dz[4];
 #pragma unroll
-    for (int it = 0; it < 4; ++it)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        float dz[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          float z = zw[(((l * 4 + it) * 4 + s) * 4 + v) * 64 + lane];
-          dz[v] = dh[it][s][v] * gelu_grad(z);
-          dzbuf[(dzrow + 16 * it + 4 * g + v) * nbp + base + 16 * s + r] = dz[v];
-        }
-        DZ.h[it][s][0] = pack2(bf16_bits(dz[0]), bf16_bits(dz[1]));
-        DZ.h[it][s][1] = pack2(bf16_bits(dz[2]), bf16_bits(dz[3]));
+      for (int v = 0; v < 4; ++v) {
+        dz[v] = dh[it][v] * gelu_grad(zl[it][0][v]);
+        dzbuf[(dzrow + 16 * it + 4 * g + v) * nbp + pos] = dz[v];
       }
+      DZ.h[it][0][0] = pack2(bf16_bits(dz[0]), bf16_bits(dz[1]));
+      DZ.h[it][0][1] = pack2(bf16_bits(dz[2]), bf16_bits(dz[3]));
+    }
   };
   auto back64 = [&](int tb) {
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       u32x4 a0 = ldtile(tiles, tb + 2 * it, lane);
       u32x4 a1 = ldtile(tiles, tb + 2 * it + 1, lane);
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        dh[it][s] = mfma(a1, bop(DZ, 1, s), mfma(a0, bop(DZ, 0, s), zero));
+      dh[it] = mfma(a1, bop(DZ, 1, 0), mfma(a0, bop(DZ, 0, 0), zero));
     }
   };
-  grad_act(2, Lay<2>::DZ);  // dZ3
-  back64(TB3);              // dH2 = W3^T dZ3
-  grad_act(1, Lay<1>::DZ);  // dZ2
-  back64(TB2);              // dH1 = W2^T dZ2
-  grad_act(0, Lay<0>::DZ);  // dZ1
+  grad_act(z[2], Lay<2>::DZ);  // dZ3
+  back64(TB3);                 // dH2 = W3^T dZ3
+  grad_act(z[1], Lay<1>::DZ);  // dZ2
+  back64(TB2);                 // dH1 = W2^T dZ2
+  grad_act(z[0], Lay<0>::DZ);  // dZ1
 
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) sse += __shfl_xor(sse, o);
   if (lane == 0) lossp[wave] = sse;
 }
 
-// Weight and bias gradient partials of layer L over one chunk of CHUNK
-// samples: dW = sum_s bf16(dZ) H^T on MFMA with the samples as the k
-// dimension, db = sum_s dZ.  part is (nchunk, NPARAM).  One wave per chunk.
+// Weight and bias gradient partials over one chunk of CHUNK samples (blockIdx.x):
+// dW = sum_s bf16(dZ) H^T on MFMA with the samples as the k dimension, db =
+// sum_s dZ.  part is (nchunk, NPARAM).  One wavefront per chunk and 16 output
+// features, all layers in one launch (blockIdx.y: four tiles of each of the
+// layers 1 to 3, then the output layer).
 template <int L>
-__global__ void __launch_bounds__(64)
-    k_mlp_dw(const uint16_t* __restrict__ hbuf, const float* __restrict__ dzbuf,
-             long long nbp, float* __restrict__ part) {
-  constexpr int IN = Lay<L>::IN, OUT = Lay<L>::OUT;
-  constexpr int NOT = (OUT + 15) / 16, NIT = (IN + 15) / 16;
+__device__ __forceinline__ void dw_tile(int ot, const uint16_t* __restrict__ hbuf,
+                                        const float* __restrict__ dzbuf, long long nbp,
+                                        float* __restrict__ part) {
+  constexpr int IN = Lay<L>::IN, OUT = Lay<L>::OUT, NIT = (IN + 15) / 16;
   const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
   const long long c = blockIdx.x;
-  f32x4 acc[NOT][NIT];
-  float dbs[NOT];
+  const int o = 16 * ot + r;
+  f32x4 acc[NIT];
+  float dbs = 0.f;
 #pragma unroll
-  for (int ot = 0; ot < NOT; ++ot) {
-    dbs[ot] = 0.f;
+  for (int it = 0; it < NIT; ++it) acc[it] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int it = 0; it < NIT; ++it) acc[ot][it] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
   for (int ks = 0; ks < CHUNK / 32; ++ks) {
     const long long p0 = c * CHUNK + 32 * ks + 8 * g;
-    u32x4 A[NOT], B[NIT];
+    u32x4 A = u32x4{0u, 0u, 0u, 0u};
+    if (o < OUT) {
+      const f32x4* src = reinterpret_cast<const f32x4*>(dzbuf + (Lay<L>::DZ + o) * nbp + p0);
+      f32x4 lo = src[0], hi = src[1];
 #pragma unroll
-    for (int ot = 0; ot < NOT; ++ot) {
-      const int o = 16 * ot + r;
-      if (o < OUT) {
-        const f32x4* src =
-            reinterpret_cast<const f32x4*>(dzbuf + (Lay<L>::DZ + o) * nbp + p0);
-        f32x4 lo = src[0], hi = src[1];
-        float sacc = dbs[ot];
+      for (int v = 0; v < 4; ++v) dbs += lo[v];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) sacc += lo[v];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) sacc += hi[v];
-        dbs[ot] = sacc;
-        A[ot] = u32x4{pack2(bf16_bits(lo[0]), bf16_bits(lo[1])),
-                      pack2(bf16_bits(lo[2]), bf16_bits(lo[3])),
-                      pack2(bf16_bits(hi[0]), bf16_bits(hi[1])),
-                      pack2(bf16_bits(hi[2]), bf16_bits(hi[3]))};
-      } else {
-        A[ot] = u32x4{0u, 0u, 0u, 0u};
-      }
+      for (int v = 0; v < 4; ++v) dbs += hi[v];
+      A = u32x4{pack2(bf16_bits(lo[0]), bf16_bits(lo[1])),
+                pack2(bf16_bits(lo[2]), bf16_bits(lo[3])),
+                pack2(bf16_bits(hi[0]), bf16_bits(hi[1])),
+                pack2(bf16_bits(hi[2]), bf16_bits(hi[3]))};
     }
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
       const int i = 16 * it + r;
-      B[it] = (i < IN) ? *reinterpret_cast<const u32x4*>(
-                             hbuf + (Lay<L>::H + i) * nbp + p0)
-                       : u32x4{0u, 0u, 0u, 0u};
+      const u32x4 B = (i < IN) ? *reinterpret_cast<const u32x4*>(
+                                     hbuf + (Lay<L>::H + i) * nbp + p0)
+                               : u32x4{0u, 0u, 0u, 0u};
+      acc[it] = mfma(A, B, acc[it]);
     }
-#pragma unroll
-    for (int ot = 0; ot < NOT; ++ot)
-#pragma unroll
-      for (int it = 0; it < NIT; ++it) acc[ot][it] = mfma(A[ot], B[it], acc[ot][it]);
   }
   float* pc = part + c * NPARAM;
 #pragma unroll
-  for (int ot = 0; ot < NOT; ++ot)
+  for (int it = 0; it < NIT; ++it)
 #pragma unroll
-    for (int it = 0; it < NIT; ++it)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int o = 16 * ot + 4 * g + v, i = 16 * it + r;
-        if (o < OUT && i < IN) pc[Lay<L>::W + o * IN + i] = acc[ot][it][v];
-      }
-#pragma unroll
-  for (int ot = 0; ot < NOT; ++ot) {
-    float s = dbs[ot];
-    s += __shfl_xor(s, 16);
-    s += __shfl_xor(s, 32);
-    if (g == 0 && 16 * ot + r < OUT) pc[Lay<L>::B + 16 * ot + r] = s;
-  }
+    for (int v = 0; v < 4; ++v) {
+      const int ow = 16 * ot + 4 * g + v, i = 16 * it + r;
+      if (ow < OUT && i < IN) pc[Lay<L>::W + ow * IN + i] = acc[it][v];
+    }
+  dbs += __shfl_xor(dbs, 16);
+  dbs += __shfl_xor(dbs, 32);
+  if (g == 0 && o < OUT) pc[Lay<L>::B + o] = dbs;
+}
+
+constexpr int DW_TILES = 13;
+__global__ void __launch_bounds__(64)
+    k_mlp_dw(const uint16_t* __restrict__ hbuf, const float* __restrict__ dzbuf,
+             long long nbp, float* __restrict__ part) {
+  const int t = blockIdx.y;
+  if (t < 4)
+    dw_tile<0>(t, hbuf, dzbuf, nbp, part);
+  else if (t < 8)
+    dw_tile<1>(t - 4, hbuf, dzbuf, nbp, part);
+  else if (t < 12)
+    dw_tile<2>(t - 8, hbuf, dzbuf, nbp, part);
+  else
+    dw_tile<3>(0, hbuf, dzbuf, nbp, part);
 }
 
 // grad = sum of the chunk partials in chunk order; loss = sum of the wave
-// partials times inv_n3 (written by thread 0).
+// partials times inv_n3, by the last block: each lane its share in order,
+// then the 256 shares pairwise.
 __global__ void __launch_bounds__(256)
     k_mlp_reduce(const float* __restrict__ part, int nchunk,
                  const float* __restrict__ lossp, int nwave, float inv_n3,
                  float* __restrict__ grad, float* __restrict__ loss) {
+  if (blockIdx.x == gridDim.x - 1) {
+    __shared__ float sh[256];
+    float s = 0.f;
+    for (int w = threadIdx.x; w < nwave; w += 256) s += lossp[w];
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+      if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) *loss = sh[0] * inv_n3;
+    return;
+  }
   int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < NPARAM) {
-    float s = 0.f;
-    for (int c = 0; c < nchunk; ++c) s += part[(size_t)c * NPARAM + p];
-    grad[p] = s;
-  }
-  if (p == 0) {
-    float s = 0.f;
-    for (int w = 0; w < nwave; ++w) s += lossp[w];
-    *loss = s * inv_n3;
-  }
+  if (p >= NPARAM) return;
+  float s = 0.f;
+#pragma unroll 8
+  for (int c = 0; c < nchunk; ++c) s += part[(size_t)c * NPARAM + p];
+  grad[p] = s;
 }
 
 // Adam (Kingma & Ba 2015) on the fp32 master parameters; c1 = 1/(1-b1^t),

@@ -79,6 +79,40 @@ def test_params_round_trip_and_forward_matches_oracle(ctx):
         net.close()
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 65, 255, 257])
+def test_partly_filled_tiles_match_oracle(ctx, n):
+    """Sample counts around the tiles of 16, the blocks of 64 and the gradient
+    chunks of 256, with the bars of the full-size tests."""
+    th, rho, ie, q = moist_states()
+    x, t, _ = orl.mlp_pairs(th, rho, ie, q, 300, seed=8)
+    x, t = np.ascontiguousarray(x[:n]), np.ascontiguousarray(t[:n])
+    net = cm.Mlp(ctx, seed=9)
+    try:
+        p = net.params()
+        y = net.forward(x)
+        yo = orl.mlp_forward(p, x, emulate=1)
+        assert np.linalg.norm(y - yo) < 1e-3 * np.linalg.norm(yo)
+        g, loss = net.loss_grad(x, t)
+        go, lo = orl.mlp_loss_grad(p, x, t, emulate=1)
+        assert abs(loss - lo) <= 1e-4 * lo
+        assert np.linalg.norm(g - go) < 1e-2 * np.linalg.norm(go)
+    finally:
+        net.close()
+
+
+def test_forward_is_the_same_on_both_sides_of_the_tile_rule(ctx):
+    """One and four sample tiles per wavefront: the same products per sample."""
+    rng = np.random.default_rng(4)
+    x = rng.uniform(-1, 1, ((1 << 21) + 1, 4)).astype(np.float32)
+    net = cm.Mlp(ctx, seed=3)
+    try:
+        y = net.forward(x)
+        np.testing.assert_array_equal(y[:70001], net.forward(x[:70001]))
+        np.testing.assert_array_equal(y[-5:], net.forward(x[-5:]))
+    finally:
+        net.close()
+
+
 def test_gradient_matches_oracle(ctx):
     th, rho, ie, q = moist_states()
     x, t, _ = orl.mlp_pairs(th, rho, ie, q, 1000, seed=4)
