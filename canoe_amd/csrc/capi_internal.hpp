@@ -20,6 +20,10 @@ struct cg_ctx {
   // Device address of this device's fixed scratch array (the implicit
   // solve's entry point that allocates nothing); null if the lookup failed.
   double* fixed_scratch = nullptr;
+  // Pinned buffers of copy_to_host, allocated by its first large copy and
+  // freed with the context.
+  void* stage[2] = {nullptr, nullptr};
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};
   char err[512] = {0};
 };
 
@@ -106,6 +110,10 @@ inline int check_status(cg_ctx* ctx) {
   }
   return CG_OK;
 }
+
+// Copy of a device array to pageable host memory after the work queued on the
+// context's stream; returns when the host array is filled (capi.hip).
+int copy_to_host(cg_ctx* ctx, void* dst, const void* src, size_t bytes);
 
 // Guided saturation adjustment of a run's resident interior cells (mlp.hip).
 int launch_satadj_run_mlp(int nmass, const cg::KGrid& g, const cg::KThermo& th,

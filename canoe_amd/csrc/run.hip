@@ -596,10 +596,7 @@ int run_download(cg_run* r, const RunBlock& b, const double* src, double* host) 
   k_relayout<<<nblk((long long)nc, 256), 256, 0, ctx->stream>>>(b.g, b.ga, r->N, src,
                                                                tmp);
   HIPCHK(ctx, hipGetLastError());
-  HIPCHK(ctx, hipMemcpyAsync(host, tmp, sizeof(double) * nc, hipMemcpyDeviceToHost,
-                             ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  return CG_OK;
+  return copy_to_host(ctx, host, tmp, sizeof(double) * nc);
 }
 
 template <int NM>
