@@ -814,12 +814,13 @@ int cg_batch_create(cg_ctx* ctx, int nblocks, const cg_block* blks,
     rb.ga = make_grid(blks[b], 0);
     ok = alloc_block(rb, r->N, *cfg);
   }
-  // workgroups per block of the time-step reduction: about 16 cells per
-  // thread in the largest block, at most 1024
+  // workgroups per block of the time-step reduction: a cell per thread up to
+  // 1,024 of them, then more (the 32,768 cells of a small 2D block at 16 per
+  // thread gave 8 workgroups and took 22 us)
   long long maxcells = 1;
   for (const RunBlock& rb : r->blocks)
     maxcells = std::max(maxcells, (long long)rb.g.nx1 * rb.g.nx2 * rb.g.nx3);
-  r->dt_parts = (int)std::min(1024LL, std::max(1LL, maxcells / (256 * 16)));
+  r->dt_parts = (int)std::min(1024LL, std::max(1LL, maxcells / 256));
   ok = ok && hipMalloc((void**)&r->part, sizeof(double) * 1024 * 8) == hipSuccess &&
        hipMalloc((void**)&r->d_dt, sizeof(double) * 3) == hipSuccess &&
        hipMemset(r->d_dt, 0, sizeof(double) * 3) == hipSuccess &&
