@@ -189,13 +189,18 @@ inline KLines make_lines(const KGrid& g, int dir) {
 }
 
 // Eight lanes per line where the lines are few.  A round of 8,192 lines (8 per
-// wavefront, a wavefront per SIMD of 256 compute units) takes about 2.2 us
-// per level, the one-lane kernels 5.5 us per level for any number of lines
-// up to 65,536 and then their memory time (5 x 5 blocks, stage of a run, 128
-// levels: 9,216 columns 0.54 against 0.72 ms, 16,384 columns 0.66 against
-// 0.74, 25,600 columns 1.17 against 0.84; 3 x 3: 9,216 columns 0.29 against
-// 0.40, 16,384 columns 0.42 against 0.41): two rounds.
-constexpr long long ROWS_MAX_LINES = 16384;
+// wavefront, a wavefront per SIMD of 256 compute units) takes 20 to 40 us and
+// 2 to 2.5 us per level, the one-lane kernels 5.5 to 6.5 us per level (5 x 5;
+// 3 to 4 us for 3 x 3) for any number of lines up to 65,536 and then their
+// memory time.  One round is faster at every measured height; a second one
+// pays where the column is tall enough for its fixed part (stage of a run,
+// 5 x 5: 16,384 columns of 128 levels 0.66 against 0.74 ms, 9,000 of 40 0.206
+// against 0.233, 16,384 of 16 0.160 against 0.104; 3 x 3: 9,216 of 128 0.29
+// against 0.40, 16,384 of 128 0.42 against 0.41, 16,384 of 16 0.125 against
+// 0.065).
+inline bool few_lines(long long nline, int n, int B) {
+  return nline <= 8192 || (n >= 40 && nline <= (B == 5 ? 16384 : 12288));
+}
 // Periodic lines: about 4.4 us per level and round of 8,192 lines (5 x 5)
 // against 17 to 22 us per level for any number up to 32,768 in the one-lane
 // kernel, whose 65,536 lines would take no longer.  x2 lines of 64 x 128 x
@@ -204,6 +209,7 @@ constexpr long long ROWS_MAX_LINES = 16384;
 // 0.66 ms.
 constexpr long long rows_max_periodic(int B) { return B == 5 ? 32768 : 16384; }
 
+// Workgroups of the row kernels.
 inline unsigned rows_grid(long long nline) { return nblk(nline, RLINES * RWAVES); }
 
 // The x1 columns of caller arrays, eight lanes per column at every size: in
@@ -256,7 +262,7 @@ void launch_lines_d(const KLines& L, const KThermo& th, double dt, const double*
                     bool per, double* du, const double* w, double* lv, int* status,
                     hipStream_t s, KTimer* tm) {
   const unsigned nb = nblk(L.nline, 64);
-  if (!per && L.nline <= ROWS_MAX_LINES)
+  if (!per && few_lines(L.nline, L.n, B))
     TIMED(tm, KID_LINES,
           (k_rows_walls<NM, B, DIR><<<rows_grid(L.nline), 64 * RWAVES, 0, s>>>(
               L, th, dt, dtp, true, true, w, du, lv, status)));

@@ -73,6 +73,8 @@ struct cg_run {
   KBlockPtr* d_bp = nullptr;
   KGroup* d_grp = nullptr;
   int ngroups = 0;
+  long long ncol = 0;  // columns of every block, and the tallest one's cells
+  int max_nx1 = 0;
   cg_tune tune;
   int ncu = 256;
   double* part = nullptr;
@@ -93,6 +95,7 @@ struct cg_run {
   // (tile_variant, tile_seg)
   KTile* d_tiles = nullptr;
   int ntiles = 0, tile_variant = -1, tile_seg = -1;
+  bool tile_fill = false;  // FP64 tiles are well filled, or few (fused_tiles)
   unsigned bc2_grid = 1, bc3_grid = 1;  // workgroups per block of the ghost kernels
   KTimer tm;
   SphRun* sph = nullptr;  // cubed-sphere run (cg_sphere_create)
@@ -120,10 +123,14 @@ void free_block(RunBlock& b) {
 // (256 x 256 x 128: 1.22 ms per stage against 1.57 for the per-face kernels
 // and the divergence).  With three species the FP64 tile needs 59 KB and one
 // wavefront per SIMD: 75 x 130 x 97 cells 0.47 ms against 0.32 for the
-// per-face kernels, which stay.
+// per-face kernels, which stay; so do they where 32 x 8 tiles are poorly
+// filled (tile_fill: 40 x 40 columns of 100 levels at 0.63 take 83 us against
+// 49 us, 100 x 90 of 40 at 0.73 118 against 89, 96 x 80 of 64 at 1 90 against
+// 110) and yet more than one level of one per compute unit (16 x 16 columns
+// of 20 levels at 0.5: 18 us in one launch against 25 in four).
 bool fused_tiles(const cg_run* r) {
   if (r->sph) return false;
-  if (r->cfg.precision == CG_PREC_FP64) return r->N == 5;
+  if (r->cfg.precision == CG_PREC_FP64) return r->N == 5 && r->tile_fill;
   return r->tune.face_variant == 3 || r->tune.face_variant == 4;
 }
 
@@ -162,11 +169,11 @@ unsigned implicit_grid(const cg_run* r) {
 }
 
 // The default launch shape of the column solve takes eight lanes per column
-// where the run has few of them (ROWS_MAX_LINES); any other shape, and every
+// where the run has few of them (few_lines); any other shape, and every
 // autotune candidate but the default, is the one-lane kernel it names.
 bool rows_columns(const cg_run* r) {
   return r->tune.implicit_wpb == 1 && r->tune.implicit_grid == 0 && r->tune.implicit_fused &&
-         r->ngroups * 64LL <= ROWS_MAX_LINES;
+         few_lines(r->ncol, r->max_nx1, (r->cfg.implicit_flag & 8) ? 5 : 3);
 }
 
 // beta: the stage weight; the sweep's step is beta times the device step.
@@ -641,9 +648,11 @@ int ensure_tiles(cg_run* r) {
   if (!fused_tiles(r)) return CG_OK;
   int tj, tk;
   tile_shape(r, tj, tk);
-  // A segment is at most march_seg levels, and short enough that the tiles
-  // fill the chip four times over (a segment's first x1 face is its only
-  // extra work).
+  // A segment is at most march_seg levels.  Where the chip's workgroup slots
+  // (by their LDS: 69 KB per FP64 tile, 72 or 45 KB per FP32 one) could take
+  // the whole run at shorter segments, the length is the one of the fewest
+  // level times: rounds of the slots times the segment and what its first x1
+  // face and tile loads cost, about half a level.
   long long per_level = 0;
   for (const RunBlock& rb : r->blocks) {
     const KGrid& g = rb.g;
@@ -651,8 +660,26 @@ int ensure_tiles(cg_run* r) {
     const long long nt = ((g.nx2 + tj - 1) / tj) * (long long)((g.nx3 + tk - 1) / tk);
     per_level += nt * g.nx1;
   }
-  const long long want = 4LL * r->ncu;
-  const int seg = (int)std::max(1LL, std::min<long long>(r->tune.march_seg, per_level / want));
+  const bool three = r->cfg.precision == CG_PREC_FP32 && r->N == 5;
+  const long long slots = (three ? 3LL : 2LL) * r->ncu;
+  int seg = std::max(1, r->tune.march_seg);
+  if (per_level < seg * slots) {
+    double best = 0.0;
+    for (int m = seg; m >= 1; --m) {
+      long long nt = 0;
+      for (const RunBlock& rb : r->blocks) {
+        const KGrid& g = rb.g;
+        if (!(g.f2 && g.f3)) continue;
+        nt += ((g.nx2 + tj - 1) / tj) * (long long)((g.nx3 + tk - 1) / tk) *
+              ((g.nx1 + m - 1) / m);
+      }
+      const double cost = (double)((nt + slots - 1) / slots) * (m + 0.6);
+      if (best == 0.0 || cost < best) {
+        best = cost;
+        seg = m;
+      }
+    }
+  }
   const int v = r->tune.face_variant;
   if (r->d_tiles && r->tile_variant == v && r->tile_seg == seg) return CG_OK;
   std::vector<int> order(r->blocks.size());
@@ -660,21 +687,29 @@ int ensure_tiles(cg_run* r) {
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
     return r->blocks[a].g.nx1 > r->blocks[b].g.nx1;
   });
-  // Workgroup w runs on XCD w % 8: each XCD gets a band of tile rows (k)
-  // of every block and level segment, so that a tile's halo neighbours
-  // mostly run on the same XCD and share its L2.  Queues of unequal length
-  // are padded with empty tiles (block -1).
+  // Workgroup w runs on XCD w % 8: each XCD gets an eighth of every block's
+  // tiles in (k, j, segment) order, a band of tile rows with all its level
+  // segments, so that a tile's halo neighbours mostly run on the same XCD and
+  // share its L2, and the XCDs' counts differ by one at most; each block
+  // starts at the shortest queue.  Queues of unequal length are padded with
+  // empty tiles (block -1).
   std::vector<KTile> q[8];
   for (int b : order) {
     const KGrid& g = r->blocks[b].g;
     if (!(g.f2 && g.f3)) continue;
     const int nbk = (g.nx3 + tk - 1) / tk;
-    for (int c0 = g.is; c0 <= g.ie; c0 += seg)
-      for (int rk = 0; rk < nbk; ++rk) {
-        const int x = (int)((long long)rk * 8 / nbk);
-        for (int j0 = g.js; j0 <= g.je; j0 += tj)
-          q[x].push_back(KTile{b, j0, g.ks + rk * tk, c0, std::min(c0 + seg, g.ie + 1)});
-      }
+    int x0 = 0;
+    for (int x = 1; x < 8; ++x)
+      if (q[x].size() < q[x0].size()) x0 = x;
+    const int nbj = (g.nx2 + tj - 1) / tj, nseg = (g.nx1 + seg - 1) / seg;
+    for (int sg = 0; sg < nseg; ++sg)
+      for (int rk = 0; rk < nbk; ++rk)
+        for (int rj = 0; rj < nbj; ++rj) {
+          const long long at = ((long long)rk * nbj + rj) * nseg + sg;
+          const int x = (int)(at * 8 / ((long long)nbk * nbj * nseg)), c0 = g.is + sg * seg;
+          q[(x0 + x) % 8].push_back(KTile{b, g.js + rj * tj, g.ks + rk * tk, c0,
+                               std::min(c0 + seg, g.ie + 1)});
+        }
   }
   size_t qmax = 0;
   for (int x = 0; x < 8; ++x) qmax = std::max(qmax, q[x].size());
@@ -804,6 +839,17 @@ int cg_batch_create(cg_ctx* ctx, int nblocks, const cg_block* blks,
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, ctx->device) == hipSuccess && prop.multiProcessorCount > 0)
     r->ncu = prop.multiProcessorCount;
+  {
+    long long cells = 0, slots = 0;
+    for (int b = 0; b < nblocks; ++b) {
+      const cg_block& k = blks[b];
+      if (k.nx2 == 1 || k.nx3 == 1) continue;
+      cells += (long long)k.nx1 * k.nx2 * k.nx3;
+      slots += (long long)k.nx1 * ((k.nx2 + F64_TJ - 1) / F64_TJ * F64_TJ) *
+               ((k.nx3 + F64_TK - 1) / F64_TK * F64_TK);
+    }
+    r->tile_fill = 5 * cells >= 4 * slots || slots <= (long long)r->ncu * F64_TJ * F64_TK;
+  }
   r->blocks.resize(nblocks);
   bool ok = true;
   for (int b = 0; b < nblocks && ok; ++b) {
@@ -812,6 +858,8 @@ int cg_batch_create(cg_ctx* ctx, int nblocks, const cg_block* blks,
     rb.g = make_grid(blks[b], 1);
     rb.g.status = ctx->d_status;  // face checks of the flux kernels
     rb.ga = make_grid(blks[b], 0);
+    r->ncol += (long long)blks[b].nx2 * blks[b].nx3;
+    r->max_nx1 = std::max(r->max_nx1, blks[b].nx1);
     ok = alloc_block(rb, r->N, *cfg);
   }
   // workgroups per block of the time-step reduction: a cell per thread up to
