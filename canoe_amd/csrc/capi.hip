@@ -97,9 +97,16 @@ namespace cg_host {
 // the device, eight threads move the other to its place.  A host array that
 // is written for the first time is bound by the page faults of the thread
 // that writes it (about 9 GB/s for one), not by the link.  Below 4 MiB the
-// runtime's own copy is as fast.
+// runtime's own copy is as fast.  Threads that share a context take turns at
+// its buffers.
 int copy_to_host(cg_ctx* ctx, void* dst, const void* src, size_t bytes) {
-  if (bytes < (4u << 20) || !ensure_stage(ctx)) {
+  std::unique_lock<std::mutex> lk(ctx->stage_mu, std::defer_lock);
+  bool staged = bytes >= (4u << 20);
+  if (staged) {
+    lk.lock();
+    staged = ensure_stage(ctx);
+  }
+  if (!staged) {
     HIPCHK(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     return CG_OK;

@@ -8,6 +8,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 
 #include "../../include/canoe_gpu.h"
 #include "cg_physics.hpp"
@@ -21,7 +22,8 @@ struct cg_ctx {
   // solve's entry point that allocates nothing); null if the lookup failed.
   double* fixed_scratch = nullptr;
   // Pinned buffers of copy_to_host, allocated by its first large copy and
-  // freed with the context.
+  // freed with the context; one copy at a time holds them.
+  std::mutex stage_mu;
   void* stage[2] = {nullptr, nullptr};
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   char err[512] = {0};
