@@ -811,8 +811,7 @@ __device__ __forceinline__ void mix_fused_tile(
 #pragma unroll
   for (int m = LO; m <= HI; ++m) load1(m, c0 - 3 + m);
   float fm[N];
-  face1(c0, fm);
-  double pfm = psf[pc + c0 * g.ps_i];
+  double pfm = 0.0;
 
   auto recon = [&](float a, float b, float c, float d, float e, float* qm,
                    float* qp) {
@@ -823,106 +822,113 @@ __device__ __forceinline__ void mix_fused_tile(
       *qm = plm_up_f(d, c, b);
     }
   };
-  for (int i = c0; i < c1; ++i) {
-    const double prd = pref[i];
-    // the own column's next x1 window cell: its loads are issued here so
-    // that they complete during the plane phases
-    const int inew = i + 1 - 3 + HI;
-    double wn[N], psvn = 0.0;
-#pragma unroll
-    for (int n = 0; n < N; ++n) wn[n] = w[colb + n * g.c.n + (long long)inew * g.c.i];
-    if (decomp) psvn = psv[pc + inew * g.ps_i];
+  // The march starts at the segment's lowest face (i = c0 - 1, no level of
+  // its own): every x1 face of a tile comes from the one copy of its
+  // arithmetic in the loop.  Two copies need not be contracted alike, and the
+  // face that two segments share has to have the same flux in both.
+#pragma clang loop unroll(disable)
+  for (int i = c0 - 1; i < c1; ++i) {
     const double pfp = psf[pc + (i + 1) * g.ps_i];
-    // (1) the level-i plane of the tile with its halo
+    if (i >= c0) {
+      const double prd = pref[i];
+      // the own column's next x1 window cell: its loads are issued here so
+      // that they complete during the plane phases
+      const int inew = i + 1 - 3 + HI;
+      double wn[N], psvn = 0.0;
 #pragma unroll
-    for (int m = 0; m < NPL; ++m) {
-      const int e = t + m * NT;
-      if (e < NP) {
-        const long long c = pbase[m] + (long long)i * g.c.i;
-        float* pl = &plane[0][0][0] + e;
+      for (int n = 0; n < N; ++n) wn[n] = w[colb + n * g.c.n + (long long)inew * g.c.i];
+      if (decomp) psvn = psv[pc + inew * g.ps_i];
+      // (1) the level-i plane of the tile with its halo
 #pragma unroll
-        for (int n = 0; n < N; ++n) {
-          double v = w[c + n * g.c.n];
-          if (n == IPR) v -= prd;
-          pl[n * NP] = (float)v;
+      for (int m = 0; m < NPL; ++m) {
+        const int e = t + m * NT;
+        if (e < NP) {
+          const long long c = pbase[m] + (long long)i * g.c.i;
+          float* pl = &plane[0][0][0] + e;
+#pragma unroll
+          for (int n = 0; n < N; ++n) {
+            double v = w[c + n * g.c.n];
+            if (n == IPR) v -= prd;
+            pl[n * NP] = (float)v;
+          }
         }
       }
-    }
-    __syncthreads();
-    // (2) face states: x2 for cells j0-1 .. j0+FT_J of the interior rows,
-    //     x3 for cells k0-1 .. k0+FT_K of the interior columns, as two item
-    //     loops with the direction's strides known at compile time; the x3
-    //     items start one wavefront further on, so that the wavefront that
-    //     took the x2 remainder is not also given the x3 remainder (no
-    //     wavefront does more than one item beyond the even share).  The
-    //     velocity slots are rotated so that the normal component comes
-    //     first (x2: v2, v3, v1; x3: v3, v1, v2), the order in which the
-    //     Riemann solver of that direction reads them: one code path serves
-    //     both directions.
-    auto states = [&](auto dirc, int e, int pj, int pk) {
-      constexpr int D = decltype(dirc)::value;  // 1: x2, 2: x3
-      constexpr int st = (D == 1) ? 1 : FT_PJ;
-      const float* pc0 = &plane[0][pk][pj];
+      __syncthreads();
+      // (2) face states: x2 for cells j0-1 .. j0+FT_J of the interior rows,
+      //     x3 for cells k0-1 .. k0+FT_K of the interior columns, as two item
+      //     loops with the direction's strides known at compile time; the x3
+      //     items start one wavefront further on, so that the wavefront that
+      //     took the x2 remainder is not also given the x3 remainder (no
+      //     wavefront does more than one item beyond the even share).  The
+      //     velocity slots are rotated so that the normal component comes
+      //     first (x2: v2, v3, v1; x3: v3, v1, v2), the order in which the
+      //     Riemann solver of that direction reads them: one code path serves
+      //     both directions.
+      auto states = [&](auto dirc, int e, int pj, int pk) {
+        constexpr int D = decltype(dirc)::value;  // 1: x2, 2: x3
+        constexpr int st = (D == 1) ? 1 : FT_PJ;
+        const float* pc0 = &plane[0][pk][pj];
 #pragma unroll
-      for (int n = 0; n < N; ++n) {
-        const int sv = (n >= IVX && n < IVX + 3) ? IVX + (n - IVX + D) % 3 : n;
-        const float* pv = pc0 + sv * (FT_PK * FT_PJ);
-        float qm, qp;
-        recon(pv[-2 * st], pv[-st], pv[0], pv[st], pv[2 * st], &qm, &qp);
-        L.qm[n][e] = qm;
-        L.qp[n][e] = qp;
+        for (int n = 0; n < N; ++n) {
+          const int sv = (n >= IVX && n < IVX + 3) ? IVX + (n - IVX + D) % 3 : n;
+          const float* pv = pc0 + sv * (FT_PK * FT_PJ);
+          float qm, qp;
+          recon(pv[-2 * st], pv[-st], pv[0], pv[st], pv[2 * st], &qm, &qp);
+          L.qm[n][e] = qm;
+          L.qp[n][e] = qp;
+        }
+      };
+      for (int e = t; e < NQ2; e += NT)
+        states(std::integral_constant<int, 1>(), e, (e % C2) + FT_H - 1, (e / C2) + FT_H);
+      {
+        constexpr int R2 = ((NQ2 % NT) + 63) / 64 * 64;
+        for (int e3 = (t + NT - R2) % NT; e3 < NQ - NQ2; e3 += NT)
+          states(std::integral_constant<int, 2>(), NQ2 + e3, (e3 % FT_J) + FT_H,
+                 (e3 / FT_J) + FT_H - 1);
       }
-    };
-    for (int e = t; e < NQ2; e += NT)
-      states(std::integral_constant<int, 1>(), e, (e % C2) + FT_H - 1, (e / C2) + FT_H);
-    {
-      constexpr int R2 = ((NQ2 % NT) + 63) / 64 * 64;
-      for (int e3 = (t + NT - R2) % NT; e3 < NQ - NQ2; e3 += NT)
-        states(std::integral_constant<int, 2>(), NQ2 + e3, (e3 % FT_J) + FT_H,
-               (e3 / FT_J) + FT_H - 1);
-    }
-    __syncthreads();
-    // (3) x2 / x3 Riemann fluxes of the tile's faces, one item list
-    for (int e = t; e < NF; e += NT) {
-      const bool x2 = e < NF2;
-      const int e3 = e - NF2;
-      const int lq = x2 ? (e / (FT_J + 1)) * C2 + e % (FT_J + 1) : NQ2 + e3;
-      const int rq = lq + (x2 ? 1 : FT_J);
-      float wl[N], wr[N], fx[N];
+      __syncthreads();
+      // (3) x2 / x3 Riemann fluxes of the tile's faces, one item list
+      for (int e = t; e < NF; e += NT) {
+        const bool x2 = e < NF2;
+        const int e3 = e - NF2;
+        const int lq = x2 ? (e / (FT_J + 1)) * C2 + e % (FT_J + 1) : NQ2 + e3;
+        const int rq = lq + (x2 ? 1 : FT_J);
+        float wl[N], wr[N], fx[N];
 #pragma unroll
-      for (int n = 0; n < N; ++n) {
-        wl[n] = L.qp[n][lq];
-        wr[n] = L.qm[n][rq];
+        for (int n = 0; n < N; ++n) {
+          wl[n] = L.qp[n][lq];
+          wr[n] = L.qm[n][rq];
+        }
+        face_check<NM, float>(g.status, wl, wr, (float)prd);
+        riemann_p<NM, 0>(th, rsolver, wl, wr, (float)prd, fx);
+#pragma unroll
+        for (int n = 0; n < N; ++n) L.fx[n][e] = fx[n];
       }
-      face_check<NM, float>(g.status, wl, wr, (float)prd);
-      riemann_p<NM, 0>(th, rsolver, wl, wr, (float)prd, fx);
+      __syncthreads();
+      // (4) x1 face i+1 in registers, the cell's divergence and sources
 #pragma unroll
-      for (int n = 0; n < N; ++n) L.fx[n][e] = fx[n];
-    }
-    __syncthreads();
-    // (4) x1 face i+1 in registers, the cell's divergence and sources
+      for (int m = LO; m < HI; ++m) {
 #pragma unroll
-    for (int m = LO; m < HI; ++m) {
+        for (int n = 0; n < N; ++n) q[n][m] = q[n][m + 1];
+        rdv[m] = rdv[m + 1];
+      }
 #pragma unroll
-      for (int n = 0; n < N; ++n) q[n][m] = q[n][m + 1];
-      rdv[m] = rdv[m + 1];
-    }
-#pragma unroll
-    for (int n = 0; n < N; ++n) q[n][HI] = (float)wn[n];
-    if (decomp) {
-      if (decomp_cell(g, inew) != inew) {  // outflow ghost
-        rdv[HI] = (float)decomp32<NM>(g, th, w, colb, psv, pc, inew, wn,
-                                      q[0][HI], q[IPR][HI]);
-      } else {
-        double r = decomp_r<NM>(th, wn);
-        rdv[HI] = (float)r;
-        q[0][HI] = fdiv((float)wn[IPR], (float)wn[0] * (float)r);
-        q[IPR][HI] = (float)(wn[IPR] - psvn);
+      for (int n = 0; n < N; ++n) q[n][HI] = (float)wn[n];
+      if (decomp) {
+        if (decomp_cell(g, inew) != inew) {  // outflow ghost
+          rdv[HI] = (float)decomp32<NM>(g, th, w, colb, psv, pc, inew, wn,
+                                        q[0][HI], q[IPR][HI]);
+        } else {
+          double r = decomp_r<NM>(th, wn);
+          rdv[HI] = (float)r;
+          q[0][HI] = fdiv((float)wn[IPR], (float)wn[0] * (float)r);
+          q[IPR][HI] = (float)(wn[IPR] - psvn);
+        }
       }
     }
     float fp[N];
     face1(i + 1, fp);
-    if (own) {
+    if (own && i >= c0) {
       double d[N];
 #pragma unroll
       for (int n = 0; n < N; ++n) {

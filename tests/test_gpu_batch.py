@@ -8,7 +8,7 @@ import pytest
 
 import canoe_amd as ca
 import oracle_lib as orl
-from helpers import cfl_dt, relerr
+from helpers import cfl_dt, perturbed_state, relerr
 
 pytestmark = pytest.mark.gpu
 
@@ -170,3 +170,24 @@ def test_batch_tiles_equal_single_block_runs_mixed(ctx, variant):
     for i, b in enumerate(bl):
         us = _run_batch(ctx, [b], dt, 2, prec=ca.PREC_FP32, tune=tune)[0]
         np.testing.assert_array_equal(ub[i], us)
+
+
+@pytest.mark.parametrize("config", [2, 4])
+@pytest.mark.parametrize("variant", [3, 4])
+def test_tiled_block_is_the_same_beside_a_large_one(ctx, config, variant):
+    """The companion's tiles change the length of the segments of levels that
+    the FP32-flux form's tiles march (one level alone, ten beside 128 x 128
+    columns of 64 levels): the block's own numbers stay the same bit for bit,
+    dry and with species."""
+    bl = []
+    for dims in ((40, 40, 40), (64, 128, 128)):
+        blk, th, cfg, w = perturbed_state(config, dims, vel=1.0, dp=1e-3)
+        bl.append((blk, th, cfg, w))
+    dt = min(cfl_dt(b[0], b[1], b[2], b[3], 0.5) for b in bl)
+    _say("beside a large block config=%d variant=%d dt=%.4f" % (config, variant, dt))
+    tune = (1, 0, 256, variant)
+    ub = _run_batch(ctx, bl, dt, 2, prec=ca.PREC_FP32, tune=tune)
+    us = _run_batch(ctx, bl[:1], dt, 2, prec=ca.PREC_FP32, tune=tune)
+    sk, sj, si = bl[0][0].interior()
+    assert np.all(np.isfinite(us[0][:, sk, sj, si]))
+    np.testing.assert_array_equal(ub[0], us[0])
