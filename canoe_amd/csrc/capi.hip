@@ -73,6 +73,17 @@ void parallel_copy(char* dst, const char* src, size_t bytes) {
     if (t.joinable()) t.join();
 }
 
+// Memory the runtime knows (page-locked, registered, managed): the copy
+// engine writes it without help.
+bool runtime_memory(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
+}
+
 bool ensure_stage(cg_ctx* ctx) {
   for (int q = 0; q < 2; ++q) {
     if (!ctx->stage[q] &&
@@ -93,15 +104,17 @@ bool ensure_stage(cg_ctx* ctx) {
 }  // namespace
 
 namespace cg_host {
-// Large copies go through two pinned buffers in turn: while one receives from
-// the device, eight threads move the other to its place.  A host array that
-// is written for the first time is bound by the page faults of the thread
-// that writes it (about 9 GB/s for one), not by the link.  Below 4 MiB the
-// runtime's own copy is as fast.  Threads that share a context take turns at
-// its buffers.
+// Large copies to pageable memory go through two pinned buffers in turn: while
+// one receives from the device, eight threads move the other to its place.  A
+// host array that is written for the first time is bound by the page faults
+// of the thread that writes it (about 9 GB/s for one), not by the link.  Below
+// 4 MiB the runtime's own copy is as fast; a page-locked array gets the direct
+// copy at any size (192 MB in 3.58 ms, 3.6 ms of processor time; through the
+// buffers 4.08 ms and 16 ms).  Threads that share a context take turns at its
+// buffers.
 int copy_to_host(cg_ctx* ctx, void* dst, const void* src, size_t bytes) {
   std::unique_lock<std::mutex> lk(ctx->stage_mu, std::defer_lock);
-  bool staged = bytes >= (4u << 20);
+  bool staged = bytes >= (4u << 20) && !runtime_memory(dst);
   if (staged) {
     lk.lock();
     staged = ensure_stage(ctx);

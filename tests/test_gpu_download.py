@@ -1,5 +1,7 @@
 """Downloads through a context's two pinned buffers: sizes around the staged
-limit (4 MiB) and the buffers (16 MiB), from several threads at once."""
+limit (4 MiB) and the buffers (16 MiB), from several threads at once; and
+downloads into page-locked memory, which do not take that way."""
+import ctypes
 import threading
 
 import numpy as np
@@ -40,3 +42,43 @@ def test_threads_share_a_context(nh):
         np.testing.assert_array_equal(got[:, sk, sj, si], w[:, sk, sj, si])
     for run in runs:
         run.close()
+
+
+def _device_file_maps():
+    """Bytes of this process's mappings of the GPU's render node, where
+    page-locked allocations of the runtime appear."""
+    n = 0
+    with open("/proc/self/maps") as f:
+        for line in f:
+            p = line.split()
+            if len(p) > 5 and p[5].startswith("/dev/dri/render"):
+                lo, hi = (int(x, 16) for x in p[0].split("-"))
+                n += hi - lo
+    return n
+
+
+@pytest.mark.parametrize("offset", [0, 24])
+def test_page_locked_arrays_are_written_directly(offset):
+    """A download into page-locked memory, whole or inside an allocation, does
+    not allocate the two staging buffers: the first download into pageable
+    memory after it still does (32 MiB of new mappings)."""
+    lib = ca.lib()
+    ctx = ca.Context(0)
+    blk, th, cfg = ca.pgen_setup(2, 64, 128, 128)
+    w = ca.pgen_init(2, 1, blk, th, cfg)
+    run = ca.Run(ctx, blk, th, cfg)
+    run.set_prim(w)
+    mem = ctypes.c_void_p()
+    assert lib.hipHostMalloc(ctypes.byref(mem), ctypes.c_size_t(w.nbytes + offset), 0) == 0
+    try:
+        dst = ctypes.cast(mem.value + offset, ctypes.POINTER(ctypes.c_double))
+        assert lib.cg_run_block_get_prim_host(run.h, 0, dst) == 0
+        got = np.ctypeslib.as_array(dst, w.shape).copy()
+        before = _device_file_maps()
+        want = run.prim()
+        assert _device_file_maps() - before >= 32 << 20
+        np.testing.assert_array_equal(got, want)
+    finally:
+        run.close()
+        ctx.close()
+        assert lib.hipHostFree(mem) == 0
