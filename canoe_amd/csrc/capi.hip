@@ -84,22 +84,27 @@ bool runtime_memory(const void* p) {
   return a.type != hipMemoryTypeUnregistered;
 }
 
+// The events are those of the context's device, which need not be the calling
+// thread's current one.
 bool ensure_stage(cg_ctx* ctx) {
-  for (int q = 0; q < 2; ++q) {
+  if (ctx->stage[0] && ctx->stage[1] && ctx->stage_ev[0] && ctx->stage_ev[1]) return true;
+  int dev = ctx->device;
+  bool ok = hipGetDevice(&dev) == hipSuccess && hipSetDevice(ctx->device) == hipSuccess;
+  for (int q = 0; q < 2 && ok; ++q) {
     if (!ctx->stage[q] &&
         hipHostMalloc(&ctx->stage[q], kStageBytes, hipHostMallocDefault) != hipSuccess) {
       ctx->stage[q] = nullptr;
-      (void)hipGetLastError();
-      return false;
+      ok = false;
     }
-    if (!ctx->stage_ev[q] &&
+    if (ok && !ctx->stage_ev[q] &&
         hipEventCreateWithFlags(&ctx->stage_ev[q], hipEventDisableTiming) != hipSuccess) {
       ctx->stage_ev[q] = nullptr;
-      (void)hipGetLastError();
-      return false;
+      ok = false;
     }
   }
-  return true;
+  (void)hipSetDevice(dev);
+  if (!ok) (void)hipGetLastError();
+  return ok;
 }
 }  // namespace
 
