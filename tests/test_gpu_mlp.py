@@ -113,6 +113,111 @@ def test_forward_is_the_same_on_both_sides_of_the_tile_rule(ctx):
         net.close()
 
 
+def _gelu64(z):
+    """tanh-form GELU, its derivative and |2 u| in 64 bits, by the sigmoid:
+    (1 + tanh u) / 2 = 1 / (1 + e^(-2u))."""
+    z = np.asarray(z, np.float64)
+    u = np.sqrt(2 / np.pi) * (z + 0.044715 * z ** 3)
+    e = np.exp(-np.clip(2 * u, -700, 700))
+    s = 1 / (1 + e)
+    dudz = np.sqrt(2 / np.pi) * (1 + 3 * 0.044715 * z * z)
+    return z * s, s + 2 * z * (e * s * s) * dudz, np.abs(2 * u)
+
+
+def _bf16(v):
+    """Round to nearest even to the upper 16 bits of a float32."""
+    b = np.asarray(v, np.float32).view(np.uint32).astype(np.uint64)
+    return ((b + 0x7fff + ((b >> 16) & 1)) >> 16 << 16).astype(np.uint32).view(np.float32)
+
+
+# parameter offsets of the four layers: weights (outputs, inputs) and biases
+W_AT, B_AT = (0, 320, 4480, 8640), (256, 4416, 8576, 8832)
+
+
+@pytest.mark.parametrize("part", ["range", "large", "nan"])
+def test_gelu_elementwise(ctx, part):
+    """The device GELU of single numbers, read through a network that adds
+    three bf16 parts of z, applies it once to that sum and passes the rounded
+    result on (a weight of 2^100 takes it where GELU is the identity or zero,
+    one unit per sign).  Bound: the bf16 number has to be that of a value
+    within 1e-6 + 6e-7 |2u| (relative) of the 64-bit one, twice what the
+    roundings of u, the 1-ulp exponential and the reciprocal add up to."""
+    rng = np.random.default_rng(11)
+    if part == "range":
+        z = rng.uniform(-9, 12, 200001).astype(np.float32)
+        small = 10.0 ** rng.uniform(-20, 0, 2000) * rng.choice([-1, 1], 2000)
+        z = np.concatenate([z, small.astype(np.float32)])
+        up = 2.0 ** 100
+    else:
+        z = (10.0 ** rng.uniform(1.1, 18, 4001) * rng.choice([-1, 1], 4001)).astype(np.float32)
+        up = 1.0
+        if part == "nan":
+            z[5::16] = np.nan
+    x = np.zeros((z.size, 4), np.float32)
+    rest = z.copy()
+    for c in range(3):  # truncated parts: their sum has no bit below z's
+        x[:, c] = (rest.view(np.uint32) & np.uint32(0xffff0000)).view(np.float32)
+        rest = (rest - x[:, c]).astype(np.float32)
+    p = np.zeros(cm.NPARAM, np.float32)
+    p[W_AT[0]:W_AT[0] + 3] = 1.0
+    p[W_AT[1]] = up
+    p[W_AT[1] + 64] = -up
+    for o in (0, 1):
+        p[W_AT[2] + o * 64 + o] = 1.0
+        p[W_AT[3] + o * 64 + o] = 1.0 / up
+    net = cm.Mlp(ctx, seed=1)
+    try:
+        net.set_params(p)
+        y = net.forward(x)
+    finally:
+        net.close()
+    bad = np.isnan(z)
+    assert np.all(np.isnan(y[bad][:, :2])) and np.all(np.isfinite(y[~bad]))
+    got, z = (y[:, 0] - y[:, 1])[~bad], z[~bad]
+    g, _, au = _gelu64(z)
+    tol = np.abs(g) * (1e-6 + 6e-7 * np.minimum(au, 100))
+    if part != "range":
+        g = np.where(z > 0, g, 0.0)
+        tol = np.where(z > 0, 0.0, 1e-30)
+    assert np.all(_bf16(g - tol) <= got) and np.all(got <= _bf16(g + tol))
+
+
+@pytest.mark.parametrize("lo,hi", [(-12.0, 12.0), (1.0, 18.0)])
+def test_gelu_derivative_elementwise(ctx, lo, hi):
+    """The device derivative of single numbers: with zero weights before it
+    and one sample, layer 3 has its biases as pre-activations, a unit output
+    weight sends the same power of two back to all of them, and the bias
+    gradients are that times the derivative in fp32.  Bound 1e-6 absolute (1.1
+    is its largest value; 16 roundings), also at |z| up to 1e18, where the
+    derivative is one or zero."""
+    rng = np.random.default_rng(12)
+    net = cm.Mlp(ctx, seed=1)
+    x = np.zeros((1, 4), np.float32)
+    worst = 0.0
+    try:
+        for n in range(200 if hi == 12.0 else 40):
+            if hi == 12.0:
+                z = rng.uniform(lo, hi, 64).astype(np.float32)
+                z[0] = 0.0
+            else:
+                z = (10.0 ** rng.uniform(lo, hi, 64)).astype(np.float32)
+                z[::4] *= -1
+            p = np.zeros(cm.NPARAM, np.float32)
+            p[B_AT[2]:B_AT[2] + 64] = z
+            p[W_AT[3]:W_AT[3] + 64] = 1.0
+            net.set_params(p)
+            y = float(net.forward(x)[0, 0])
+            back = 2.0 ** np.floor(np.log2(abs(y) + 1.0))
+            t = np.array([[y - 1.5 * back, 0, 0]], np.float32)
+            grad, _ = net.loss_grad(x, t)
+            got = grad[B_AT[2]:B_AT[2] + 64].astype(np.float64) / back
+            worst = max(worst, np.max(np.abs(got - _gelu64(z)[1])))
+    finally:
+        net.close()
+    print("derivative, z of %g..%g: largest error %.2e" % (lo, hi, worst), flush=True)
+    assert worst <= 1e-6
+
+
 def test_gradient_matches_oracle(ctx):
     th, rho, ie, q = moist_states()
     x, t, _ = orl.mlp_pairs(th, rho, ie, q, 1000, seed=4)
