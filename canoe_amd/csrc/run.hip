@@ -91,10 +91,10 @@ struct cg_run {
   double* h_dt = nullptr;
   double* dt_part = nullptr;  // per-workgroup minima, dt_parts per block
   int dt_parts = 1;
-  // tiles of the fused face kernel over every 3D block, built for
-  // (tile_variant, tile_seg)
+  // tiles of the fused face kernel over every 3D block (none in a run
+  // without them), built for (tile_variant, tile_march) of the launch shape
   KTile* d_tiles = nullptr;
-  int ntiles = 0, tile_variant = -1, tile_seg = -1;
+  int ntiles = 0, tile_variant = -1, tile_march = -1;
   bool tile_fill = false;  // FP64 tiles are well filled, or few (fused_tiles)
   unsigned bc2_grid = 1, bc3_grid = 1;  // workgroups per block of the ghost kernels
   KTimer tm;
@@ -646,6 +646,8 @@ int capture(cg_run* r) {
 // capturing).  Tiles of the tallest blocks come first.
 int ensure_tiles(cg_run* r) {
   if (!fused_tiles(r)) return CG_OK;
+  const int v = r->tune.face_variant, march = r->tune.march_seg;
+  if (r->tile_variant == v && r->tile_march == march) return CG_OK;
   int tj, tk;
   tile_shape(r, tj, tk);
   // A segment is at most march_seg levels.  Where the chip's workgroup slots
@@ -662,7 +664,7 @@ int ensure_tiles(cg_run* r) {
   }
   const bool three = r->cfg.precision == CG_PREC_FP32 && r->N == 5;
   const long long slots = (three ? 3LL : 2LL) * r->ncu;
-  int seg = std::max(1, r->tune.march_seg);
+  int seg = std::max(1, march);
   if (per_level < seg * slots) {
     double best = 0.0;
     for (int m = seg; m >= 1; --m) {
@@ -680,8 +682,6 @@ int ensure_tiles(cg_run* r) {
       }
     }
   }
-  const int v = r->tune.face_variant;
-  if (r->d_tiles && r->tile_variant == v && r->tile_seg == seg) return CG_OK;
   std::vector<int> order(r->blocks.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
@@ -719,15 +719,18 @@ int ensure_tiles(cg_run* r) {
       tiles.push_back(slot < q[x].size() ? q[x][slot] : KTile{-1, 0, 0, 0, 0});
   if (r->d_tiles) (void)hipFree(r->d_tiles);
   r->d_tiles = nullptr;
+  r->ntiles = 0;
+  r->tile_variant = r->tile_march = -1;  // tried again after a failure
+  if (!tiles.empty()) {
+    HIPCHK(r->ctx, hipMalloc((void**)&r->d_tiles, sizeof(KTile) * tiles.size()));
+    HIPCHK(r->ctx, hipMemcpy(r->d_tiles, tiles.data(), sizeof(KTile) * tiles.size(),
+                             hipMemcpyHostToDevice));
+    // the copy runs on the null stream: done before the next launch reads it
+    HIPCHK(r->ctx, hipDeviceSynchronize());
+  }
   r->ntiles = (int)tiles.size();
   r->tile_variant = v;
-  r->tile_seg = seg;
-  if (tiles.empty()) return CG_OK;
-  HIPCHK(r->ctx, hipMalloc((void**)&r->d_tiles, sizeof(KTile) * tiles.size()));
-  HIPCHK(r->ctx, hipMemcpy(r->d_tiles, tiles.data(), sizeof(KTile) * tiles.size(),
-                           hipMemcpyHostToDevice));
-  // the copy runs on the null stream: done before the next launch reads it
-  HIPCHK(r->ctx, hipDeviceSynchronize());
+  r->tile_march = march;
   return CG_OK;
 }
 
