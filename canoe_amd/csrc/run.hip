@@ -134,6 +134,9 @@ bool fused_tiles(const cg_run* r) {
   return r->tune.face_variant == 3 || r->tune.face_variant == 4;
 }
 
+// Levels of a tile's segment where the caller sets none (ensure_tiles).
+constexpr int kMarchSeg = 16;
+
 // Columns of a tile.
 constexpr int F64_TJ = 32, F64_TK = 8;
 void tile_shape(const cg_run* r, int& tj, int& tk) {
@@ -650,9 +653,10 @@ int ensure_tiles(cg_run* r) {
   if (r->tile_variant == v && r->tile_march == march) return CG_OK;
   int tj, tk;
   tile_shape(r, tj, tk);
-  // A segment is at most march_seg levels.  Where the chip's workgroup slots
-  // (by their LDS: 69 KB per FP64 tile, 72 or 45 KB per FP32 one) could take
-  // the whole run at shorter segments, the length is the one of the fewest
+  // Segments have march_seg levels as the caller set it, but for its default,
+  // which stands for at most as many: where the chip's workgroup slots (by
+  // their LDS: 69 KB per FP64 tile, 72 or 45 KB per FP32 one) could take the
+  // whole run at shorter segments, the length is then the one of the fewest
   // level times: rounds of the slots times the segment and what its first x1
   // face and tile loads cost, about half a level.
   long long per_level = 0;
@@ -665,7 +669,7 @@ int ensure_tiles(cg_run* r) {
   const bool three = r->cfg.precision == CG_PREC_FP32 && r->N == 5;
   const long long slots = (three ? 3LL : 2LL) * r->ncu;
   int seg = std::max(1, march);
-  if (per_level < seg * slots) {
+  if (march == kMarchSeg && per_level < seg * slots) {
     double best = 0.0;
     for (int m = seg; m >= 1; --m) {
       long long nt = 0;
@@ -836,7 +840,7 @@ int cg_batch_create(cg_ctx* ctx, int nblocks, const cg_block* blks,
   r->tune.implicit_grid = 0;
   r->tune.flux_block = 256;
   r->tune.face_variant = 3;
-  r->tune.march_seg = 16;
+  r->tune.march_seg = kMarchSeg;
   r->tune.implicit_fused = 1;
   r->tune.step_ms = 0.0;
   hipDeviceProp_t prop;

@@ -453,13 +453,15 @@ int cg_run_block_sums(cg_run* run, int block, double* out_host);
  * march_seg cells, x1 fused with the divergence; 2: as 1 for x2 / x3, one
  * lane per x1 face and a divergence kernel; 3 / 4: all faces and the
  * divergence in one LDS tile kernel of 32 x 8 / 16 x 16 columns marching up
- * segments of at most march_seg levels, 3D blocks only, else as 2); step_ms
- * is the step time
- * measured by the autotuner.  The default column-solve shape (1, 0, fused)
- * means eight lanes per column where the run has few columns; dry FP64 runs
- * of well filled 3D blocks take all faces and the divergence in one tile
- * kernel, which flux_block does not reach.  No counterpart in the reference
- * (CPU loop nests). */
+ * segments of march_seg levels, 3D blocks only, else as 2; of march_seg's
+ * default, 16, at most as many, by the size of the run); step_ms is the step
+ * time measured by the autotuner.  The default column-solve shape (1, 0,
+ * fused) means eight lanes per column where the run has few columns.  Dry
+ * FP64 runs whose 32 x 8 column tiles are well filled, or are few, take all
+ * faces and the divergence of their 3D blocks in one tile kernel with
+ * segments of march_seg levels by the same rule; flux_block does not reach
+ * it, and face_variant has no effect in FP64.  No counterpart in the
+ * reference (CPU loop nests). */
 typedef struct cg_tune {
   int implicit_wpb;
   int implicit_grid;
