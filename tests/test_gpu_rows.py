@@ -100,3 +100,62 @@ def test_caller_periodic_lines_equal_the_oracle(ctx, flag, dims):
     assert r == 0
     sk, sj, si = blk.interior()
     assert relerr(got[:, sk, sj, si], ref[:, sk, sj, si]) <= TOL
+
+
+# (x2 lines are nx1 x nx3 of nx2 cells, x3 lines nx1 x nx2 of nx3) on both
+# sides of the limits of the eight-lane kernels: short lines between walls
+# 8,192, periodic lines 32,768 (5 x 5) and 16,384 (3 x 3).  Walled x3 lines of
+# moist blocks this wide are refused (the shuffled species weights would lie
+# past the end of w).
+LIMITS = [(10, True, (64, 5, 128)), (10, True, (64, 5, 129)), (2, True, (64, 5, 129)),
+          (10, False, (128, 5, 256)), (10, False, (128, 5, 257)), (12, False, (257, 128, 6)),
+          (2, False, (128, 5, 128)), (2, False, (128, 5, 129)), (4, False, (129, 128, 6))]
+
+
+@pytest.mark.parametrize("config,flag,walls,dims",
+                         [(2,) + c for c in LIMITS] + [(4,) + c for c in LIMITS] +
+                         [(2, 12, True, (129, 64, 6)), (2, 4, True, (129, 64, 6))])
+def test_caller_lines_on_both_sides_of_the_limits(ctx, config, flag, walls, dims):
+    blk, th, cfg, w = perturbed_state(config, dims)
+    if walls:
+        for s in range(2, 6):
+            blk.bc[s] = ca.BC_REFLECT
+        w = ca.apply_bc_host(blk, w)
+    du = _increments(blk, 9)
+    print("limits config=%d flag=%d walls=%s dims=%s" % (config, flag, walls, dims), flush=True)
+    got = ca.ImplicitSolver(ctx, blk, th, flag).solve_implicit_3d(du, w, 0.4)
+    ref, r = orl.implicit_solve(blk, th, du, w, 0.4, flag)
+    assert r == 0
+    sk, sj, si = blk.interior()
+    assert relerr(got[:, sk, sj, si], ref[:, sk, sj, si]) <= TOL
+
+
+@pytest.mark.parametrize("flag,dims", [(10, (128, 41, 130)), (2, (96, 41, 130)),
+                                       (12, (128, 130, 41)), (4, (96, 130, 41))])
+def test_many_tall_lines_equal_the_same_lines_in_halves(ctx, flag, dims):
+    """Lines of 41 cells between walls, just above the 16,384 (5 x 5) and 12,288
+    (3 x 3) that the eight-lane kernel takes at that height: the one-lane
+    kernel's whole block equals its halves, which are below, bit for bit."""
+    blk, th, cfg, w = perturbed_state(2, dims)
+    for s in range(2, 6):
+        blk.bc[s] = ca.BC_REFLECT
+    w = ca.apply_bc_host(blk, w)
+    du = _increments(blk, 11)
+    print("halves flag=%d dims=%s" % (flag, dims), flush=True)
+    whole = ca.ImplicitSolver(ctx, blk, th, flag).solve_implicit_3d(du, w, 0.4)
+    axis = 2 if flag & 4 else 1  # arrays (n, k, j, i): cut across the lines
+    n = dims[1] if flag & 4 else dims[2]
+    hdims = list(dims)
+    hdims[1 if flag & 4 else 2] = n // 2
+    hb = perturbed_state(2, tuple(hdims))[0]
+    for q in range(6):
+        hb.bc[q] = blk.bc[q]
+    hb.dx1, hb.dx2, hb.dx3 = blk.dx1, blk.dx2, blk.dx3
+    for lo in (0, n // 2):
+        cut = [slice(None)] * 4
+        cut[axis] = slice(lo, lo + n // 2 + 6)  # with three ghosts either side
+        cut = tuple(cut)
+        half = ca.ImplicitSolver(ctx, hb, th, flag).solve_implicit_3d(
+            np.ascontiguousarray(du[cut]), np.ascontiguousarray(w[cut]), 0.4)
+        sk, sj, si = hb.interior()
+        np.testing.assert_array_equal(half[:, sk, sj, si], whole[cut][:, sk, sj, si])
