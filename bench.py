@@ -214,7 +214,7 @@ def algorithmic(blk, cfg):
 OPS = {
     "flux_divergence": ["k_hydrostatic_scan", "k_flux_x1", "k_flux_h<x2>",
                         "k_flux_h<x3>", "k_divergence", "k_flux32",
-                        "k_mix_fused"],
+                        "k_mix_fused", "k_fused64"],
     "implicit_solve": ["k_implicit_fwd", "k_implicit_bwd", "k_implicit_fused"],
     "update": ["k_update", "k_bc_x1", "k_bc_x2", "k_bc_x3",
                "k_satadj_run_mlp"],

@@ -121,9 +121,10 @@ void free_block(RunBlock& b) {
 // 3D blocks whose faces and divergence come from one tile launch per stage:
 // face variants 3 / 4 of the FP32-flux form, and the FP64 form of dry runs
 // (256 x 256 x 128: 1.22 ms per stage against 1.57 for the per-face kernels
-// and the divergence).  With three species the FP64 tile needs 59 KB and one
-// wavefront per SIMD: 75 x 130 x 97 cells 0.47 ms against 0.32 for the
-// per-face kernels, which stay; so do they where 32 x 8 tiles are poorly
+// and the divergence).  With three species a 32 x 8 tile would need 111 KB of
+// LDS; the one tried, 16 x 8 with 59 KB, has two workgroups of two wavefronts
+// per CU, one wavefront per SIMD: 75 x 130 x 97 cells 0.47 ms against 0.32 for
+// the per-face kernels, which stay; so do they where 32 x 8 tiles are poorly
 // filled (tile_fill: 40 x 40 columns of 100 levels at 0.63 take 83 us against
 // 49 us, 100 x 90 of 40 at 0.73 118 against 89, 96 x 80 of 64 at 1 90 against
 // 110) and yet more than one level of one per compute unit (16 x 16 columns
@@ -149,7 +150,7 @@ void launch_fused64(cg_run* r, const KSource& src, KTimer* tm) {
   hipStream_t s = r->ctx->stream;
   const bool w5h = r->cfg.order_h == 5, w5v = r->cfg.order_v == 5;
 #define CG_FUSED64(OH, OV)                                                           \
-  TIMED(tm, KID_DIVERGENCE,                                                          \
+  TIMED(tm, KID_MIX_FUSED,                                                           \
         (k_fused64_batch<0, OH, OV, F64_TJ, F64_TK>                                  \
              <<<(unsigned)r->ntiles, F64_TJ * F64_TK, 0, s>>>(r->d_bp, r->d_tiles, r->kt, \
                                                               src, r->cfg.rsolver)))
@@ -1181,7 +1182,9 @@ int cg_run_kernel_stats(cg_run* r, int kernel_id, double* total_ms,
   if (!r || kernel_id < 0 || kernel_id >= KID_COUNT) return CG_ERR_ARG;
   if (total_ms) *total_ms = r->tm.ms[kernel_id];
   if (launches) *launches = r->tm.cnt[kernel_id];
-  if (name) *name = kKernelNames[kernel_id];
+  // one id for the tile kernels of both forms
+  const bool f64 = kernel_id == KID_MIX_FUSED && r->cfg.precision == CG_PREC_FP64;
+  if (name) *name = f64 ? "k_fused64" : kKernelNames[kernel_id];
   return CG_OK;
 }
 
