@@ -6,8 +6,9 @@
 // Weights and layer inputs are bf16, products accumulate in fp32 on MFMA
 // (v_mfma_f32_16x16x32_bf16), everything elementwise is fp32.
 //
-// Wave-level formulation.  One wavefront carries 64 samples as 4 sample tiles
-// of 16.  Layers are evaluated transposed, Z^T = W H^T, so that W is the A
+// Wave-level formulation.  One wavefront carries S sample tiles of 16: one in
+// the gradient and in forwards of few samples, four in large forwards and the
+// guided adjustment.  Layers are evaluated transposed, Z^T = W H^T, so that W is the A
 // operand and the activations are the B operand:
 //   A (16 x 32):  lane l holds A[l % 16][8 (l / 16) + v],  v = 0..7
 //   B (32 x 16):  lane l holds B[8 (l / 16) + v][l % 16]

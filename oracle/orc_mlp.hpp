@@ -1,9 +1,9 @@
 // Oracle elementwise routines of the saturation-guess network -- TEST
 // INFRASTRUCTURE ONLY (the results are compared with it; never the product).
 //
-// The device library carries its own copy of the same algorithms, so that
-// everything outside the matrix products is evaluated identically on both
-// sides:
+// The device library has the same bf16 rounding; its GELU takes the hardware's
+// exponential and reciprocal, which the exponential below does not reproduce
+// bit for bit, so comparisons allow for single-precision rounding there.
 //   bf16:  round-to-nearest-even of an IEEE binary32 to its upper 16 bits
 //          (NaN kept quiet).
 //   exp_f: Cody-Waite reduction x = k ln2 + r with ln2 split as
