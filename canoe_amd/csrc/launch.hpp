@@ -188,50 +188,84 @@ inline KLines make_lines(const KGrid& g, int dir) {
   return L;
 }
 
-// Eight lanes per line where the lines are few.  A round of 8,192 lines (8 per
-// wavefront, a wavefront per SIMD of 256 compute units) takes 20 to 40 us and
-// 2 to 2.5 us per level, the one-lane kernels 5.5 to 6.5 us per level (5 x 5;
-// 3 to 4 us for 3 x 3) for any number of lines up to 65,536 and then their
-// memory time.  One round is faster at every measured height; a second one
-// pays where the column is tall enough for its fixed part (stage of a run,
-// 5 x 5: 16,384 columns of 128 levels 0.66 against 0.74 ms, 9,000 of 40 0.206
-// against 0.233, 16,384 of 16 0.160 against 0.104; 3 x 3: 9,216 of 128 0.29
-// against 0.40, 16,384 of 128 0.42 against 0.41, 16,384 of 16 0.125 against
-// 0.065).
-inline bool few_lines(long long nline, int n, int B) {
-  return nline <= 8192 || (n >= 40 && nline <= (B == 5 ? 16384 : 12288));
+// Eight lanes per line or one.  A round of 8,192 lines (8 per wavefront, a
+// wavefront per SIMD of 256 compute units) costs 20 to 40 us and 1 to 2.5 us
+// per level (periodic lines 4.4) with eight lanes; one lane per line costs 3
+// to 6.5 us per level (periodic 10 to 20) for any number of lines up to
+// 65,536, and its memory time where that is more, as on caller arrays, whose
+// columns it reads with a cache line per lane.  So octets win where lines are
+// few, or long enough for their fixed part.  Of each kernel: the heights from
+// which they are faster, as measured at 3 to 96 levels of 1,024 to 131,072
+// lines, at the given numbers of lines; linear between these and in
+// proportion below the first; 0 is never, and above the last number of lines
+// its height counts.
+constexpr int kEvenLines[7] = {8192, 8448, 12288, 16384, 24576, 32768, 65536};
+struct KEven {
+  int h[7];
+};
+inline bool octets(const KEven& e, long long nline, int n) {
+  if (nline <= kEvenLines[0]) return (long long)n * kEvenLines[0] >= e.h[0] * nline;
+  for (int k = 1; k < 7; ++k) {
+    if (nline > kEvenLines[k]) continue;
+    if (e.h[k] == 0) return false;
+    const double f = double(nline - kEvenLines[k - 1]) / (kEvenLines[k] - kEvenLines[k - 1]);
+    return n >= e.h[k - 1] + f * (e.h[k] - e.h[k - 1]);
+  }
+  return e.h[6] != 0 && n >= e.h[6];
 }
-// Periodic lines: about 4.4 us per level and round of 8,192 lines (5 x 5)
-// against 17 to 22 us per level for any number up to 32,768 in the one-lane
-// kernel, whose 65,536 lines would take no longer.  x2 lines of 64 x 128 x
-// 128 cells 0.63 against 2.18 ms, of 128 x 256 x 256 4.51 against 5.55 ms;
-// 3 x 3 x2 lines of 64 x 256 x 128 0.57 against 1.16, x3 lines 0.48 against
-// 0.66 ms.
-constexpr long long rows_max_periodic(int B) { return B == 5 ? 32768 : 16384; }
+// Rows: dry, with species; columns: 5 x 5, 3 x 3 blocks.
+// A stage's columns of a run, 5 x 5: 4,096 columns of 3 levels 35 us against 27
+// for one lane, of 8 45 against 49; 8,190 of 8 67 against 53, of 16 86 against
+// 95, of 64 175 against 324; 16,384 of 48 286 against 252, of 128 600 against
+// 648.  With species 12,769 of 40 274 against 258.
+constexpr KEven kRunColumns[2][2] = {{{{13, 34, 46, 90}}, {{19, 28, 57}}},
+                                     {{{10, 32, 51, 95}}, {{11, 20, 80}}}};
+// x2 / x3 lines between walls, 5 x 5 (calls of cg_implicit_solve, here and
+// below): 8,192 lines of 5 cells 92 us against 73, of 24 132 against 144, of 96 247 against 425.
+constexpr KEven kWallLines[2][2] = {{{{18, 44, 62, 70}}, {{30, 37, 56, 95}}},
+                                    {{{13, 27, 38, 49}}, {{16, 18, 33, 43}}}};
+// Periodic lines, 5 x 5: 16,384 lines of 5 cells 169 us against 98, of 48 515
+// against 840; 32,000 of 16 476 against 339, of 48 956 against 1,052.
+constexpr KEven kPeriodicLines[2][2] = {{{{7, 11, 15, 17, 24, 36}}, {{28, 33, 45, 50}}},
+                                        {{{5, 9, 11, 14, 20, 31}}, {{18, 64, 58, 56}}}};
+// x1 columns of caller arrays, 5 x 5: 262,144 columns of 5 levels 1,482 us
+// against 371, of 64 4,815 against 5,200; 65,536 of 128 2,187 against 2,712,
+// with species 2,474 against 4,750.
+constexpr KEven kCallerColumns[2][2] = {
+    {{{17, 40, 52, 54, 72, 50, 46}}, {{29, 28, 44, 60, 61, 42, 23}}},
+    {{{13, 28, 38, 39, 25, 18, 16}}, {{16, 18, 27, 40, 19, 11, 10}}}};
 
 // Workgroups of the row kernels.
 inline unsigned rows_grid(long long nline) { return nblk(nline, RLINES * RWAVES); }
 
-// The x1 columns of caller arrays, eight lanes per column at every size: in
-// the AthenaArray layout its lanes run along the column (64 bytes per octet),
-// where one lane per column put every lane of a load on a cache line of its
-// own.  256 x 256 columns of 128 levels: 2.08 ms against 2.58 (5 x 5), 1.12
-// against 2.18 ms (3 x 3); 32 x 32 columns of 128 levels 0.19 ms.
+// The x1 columns of caller arrays.  In the AthenaArray layout the eight lanes
+// of a column run along it (64 bytes per octet), where one lane per column
+// puts every lane of a load on a cache line of its own; short columns, though,
+// leave most of an octet's work to its fixed part.  One lane per column folds
+// both ends as walls, so a column with one periodic side has eight.
+template <int NM, int B>
+void launch_columns_b(const KGrid& g, const KThermo& th, double dt, double* du,
+                      const double* w, double* arch, int* status, hipStream_t s, KTimer* tm) {
+  const KLines L = make_lines(g, 0);
+  const bool flo = g.bc[0] != CG_BC_PERIODIC, fhi = g.bc[1] != CG_BC_PERIODIC;
+  if (!flo || !fhi || octets(kCallerColumns[NM > 0][B == 3], L.nline, L.n))
+    TIMED(tm, KID_IMPLICIT_FUSED,
+          (k_rows_walls<NM, B, 0><<<rows_grid(L.nline), 64 * RWAVES, 0, s>>>(
+              L, th, dt, nullptr, flo, fhi, w, du, arch, status)));
+  else
+    TIMED(tm, KID_IMPLICIT_FUSED,
+          (k_line_walls<NM, B, 0><<<nblk(L.nline, 64), 64, 0, s>>>(L, th, dt, nullptr, w, du,
+                                                                   arch, status)));
+}
+
 template <int NM>
 void launch_implicit(const KGrid& g, const KThermo& th, double dt, int flag,
                      double* du, const double* w, double* arch, int* status,
                      hipStream_t s, KTimer* tm = nullptr) {
-  const long long ncol = (long long)g.nx2 * g.nx3;
-  const bool flo = g.bc[0] != CG_BC_PERIODIC, fhi = g.bc[1] != CG_BC_PERIODIC;
-  const KLines L = make_lines(g, 0);
   if (flag & 8)
-    TIMED(tm, KID_IMPLICIT_FUSED,
-          (k_rows_walls<NM, 5, 0><<<rows_grid(ncol), 64 * RWAVES, 0, s>>>(
-              L, th, dt, nullptr, flo, fhi, w, du, arch, status)));
+    launch_columns_b<NM, 5>(g, th, dt, du, w, arch, status, s, tm);
   else
-    TIMED(tm, KID_IMPLICIT_FUSED,
-          (k_rows_walls<NM, 3, 0><<<rows_grid(ncol), 64 * RWAVES, 0, s>>>(
-              L, th, dt, nullptr, flo, fhi, w, du, arch, status)));
+    launch_columns_b<NM, 3>(g, th, dt, du, w, arch, status, s, tm);
 }
 
 template <int NM>
@@ -262,11 +296,11 @@ void launch_lines_d(const KLines& L, const KThermo& th, double dt, const double*
                     bool per, double* du, const double* w, double* lv, int* status,
                     hipStream_t s, KTimer* tm) {
   const unsigned nb = nblk(L.nline, 64);
-  if (!per && few_lines(L.nline, L.n, B))
+  if (!per && octets(kWallLines[NM > 0][B == 3], L.nline, L.n))
     TIMED(tm, KID_LINES,
           (k_rows_walls<NM, B, DIR><<<rows_grid(L.nline), 64 * RWAVES, 0, s>>>(
               L, th, dt, dtp, true, true, w, du, lv, status)));
-  else if (per && L.nline <= rows_max_periodic(B))
+  else if (per && octets(kPeriodicLines[NM > 0][B == 3], L.nline, L.n))
     TIMED(tm, KID_LINES,
           (k_rows_periodic<NM, B, DIR><<<rows_grid(L.nline), 64 * RWAVES, 0, s>>>(
               L, th, dt, dtp, w, du, lv, status)));

@@ -173,11 +173,12 @@ unsigned implicit_grid(const cg_run* r) {
 }
 
 // The default launch shape of the column solve takes eight lanes per column
-// where the run has few of them (few_lines); any other shape, and every
-// autotune candidate but the default, is the one-lane kernel it names.
+// where that is faster by the number of columns and the tallest block
+// (kRunColumns); any other shape, and every autotune candidate but the
+// default, is the one-lane kernel it names.
 bool rows_columns(const cg_run* r) {
   return r->tune.implicit_wpb == 1 && r->tune.implicit_grid == 0 && r->tune.implicit_fused &&
-         few_lines(r->ncol, r->max_nx1, (r->cfg.implicit_flag & 8) ? 5 : 3);
+         octets(kRunColumns[r->N > 5][(r->cfg.implicit_flag & 8) ? 0 : 1], r->ncol, r->max_nx1);
 }
 
 // beta: the stage weight; the sweep's step is beta times the device step.
