@@ -205,16 +205,26 @@ __global__ void __launch_bounds__(256)
 
 // psf and psv of every column of a block: 16 columns per workgroup while
 // their two LDS arrays fit 64 KB (255 cells with ghosts), 4 up to 1,023 cells,
-// one column per lane above.
+// one column per lane above.  One column per lane also where a run's layout
+// has lanes side by side in memory and columns are many for their height,
+// which grows with the square of their number (c thousands): their wavefronts
+// fill the chip, and the workgroups' barriers and partly used lanes cost more.
+// 65,536 columns of 5 levels 15 us either way, 131,072 of 8 26 us in LDS
+// against 22, of 24 44 against 45; 196,608 of 40 91 against 85, of 64 132
+// against 130; 262,144 of 12 57 against 41, of 128 392 against 290.  A caller's
+// arrays, whose lanes would be a column apart, are 1.0 to 1.2 times as fast in
+// LDS at these sizes.
 template <int NM>
 void launch_scan(const KGrid& g, const KThermo& th, const double* w, double* psf, double* psv,
                  hipStream_t s) {
   const long long ncol = (long long)g.nx2 * g.nx3;
   const size_t per = sizeof(double) * (2 * (size_t)g.nc1 + 1);
-  if (per * 16 <= 65536)
+  const long long c = ncol / 1024;
+  const bool many = g.lvl && (c >= 256 || 2048LL * g.nx1 < 3 * c * c);
+  if (per * 16 <= 65536 && !many)
     k_hydrostatic_scan_lds<NM, 16>
         <<<(unsigned)((ncol + 15) / 16), 256, per * 16, s>>>(g, th, w, psf, psv);
-  else if (per * 4 <= 65536)
+  else if (per * 4 <= 65536 && !many)
     k_hydrostatic_scan_lds<NM, 4>
         <<<(unsigned)((ncol + 3) / 4), 256, per * 4, s>>>(g, th, w, psf, psv);
   else
