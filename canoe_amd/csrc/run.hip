@@ -871,13 +871,17 @@ int cg_batch_create(cg_ctx* ctx, int nblocks, const cg_block* blks,
     r->max_nx1 = std::max(r->max_nx1, blks[b].nx1);
     ok = alloc_block(rb, r->N, *cfg);
   }
-  // workgroups per block of the time-step reduction: a cell per thread up to
-  // 1,024 of them, then more (the 32,768 cells of a small 2D block at 16 per
-  // thread gave 8 workgroups and took 22 us)
+  // workgroups per block of the time-step reduction: a cell per thread of the
+  // largest block while all blocks' fit 2,048, the chip's eight per CU (the
+  // 32,768 cells of a small 2D block at 16 per thread gave 8 workgroups and
+  // took 22 us), then fewer down to 16 cells per thread, at most 1,024: 64
+  // blocks of 64 x 64 x 32 cells 107 us per call with 32 workgroups each, 143
+  // us with 512
   long long maxcells = 1;
   for (const RunBlock& rb : r->blocks)
     maxcells = std::max(maxcells, (long long)rb.g.nx1 * rb.g.nx2 * rb.g.nx3);
-  r->dt_parts = (int)std::min(1024LL, std::max(1LL, maxcells / 256));
+  const long long wide = std::min(maxcells / 256, 2048LL / nblocks);
+  r->dt_parts = (int)std::min(1024LL, std::max({1LL, wide, maxcells / (256 * 16)}));
   ok = ok && hipMalloc((void**)&r->part, sizeof(double) * 1024 * 8) == hipSuccess &&
        hipMalloc((void**)&r->d_dt, sizeof(double) * 3) == hipSuccess &&
        hipMemset(r->d_dt, 0, sizeof(double) * 3) == hipSuccess &&

@@ -6,6 +6,8 @@ the same loop driven by the oracle.
 The step is a minimum of per-cell values computed with the same expressions
 in FP64, so any reduction order gives the same double: the bar is equality.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -206,3 +208,26 @@ def test_run_stage_rejects_bad_arguments(ctx):
                 run.stage(s, dt)
     finally:
         run.close()
+
+
+def test_new_dt_of_many_blocks_takes_no_longer_than_of_one(ctx):
+    """The same 8.4 million cells as 64 blocks and as one: the reduction does
+    not launch so many workgroups per block that their number counts (a cell
+    per thread in every block took 1.33 times as long)."""
+    best = {}
+    for nb, dims in ((64, (64, 64, 32)), (1, (64, 128, 1024))):
+        blk, th, cfg = ca.pgen_setup(2, *dims)
+        w = ca.pgen_init(2, 1, blk, th, cfg)
+        run = ca.Run(ctx, None, th, cfg, blocks=[blk] * nb)
+        try:
+            for b in range(nb):
+                run.set_prim(w, b)
+            best[nb] = np.inf
+            for _ in range(30):
+                t0 = time.perf_counter()
+                run.new_dt(0.3)
+                best[nb] = min(best[nb], time.perf_counter() - t0)
+        finally:
+            run.close()
+    print("64 blocks %.1f us, one %.1f us" % (1e6 * best[64], 1e6 * best[1]), flush=True)
+    assert best[64] <= 1.15 * best[1]
