@@ -84,13 +84,15 @@ bool runtime_memory(const void* p) {
   return a.type != hipMemoryTypeUnregistered;
 }
 
-// The events are those of the context's device, which need not be the calling
-// thread's current one.
-bool ensure_stage(cg_ctx* ctx) {
-  if (ctx->stage[0] && ctx->stage[1] && ctx->stage_ev[0] && ctx->stage_ev[1]) return true;
+// The first `count` buffers (one or two) and their events, which are those of
+// the context's device (it need not be the calling thread's current one).
+bool ensure_stage(cg_ctx* ctx, int count) {
+  bool ok = true;
+  for (int q = 0; q < count; ++q) ok = ok && ctx->stage[q] && ctx->stage_ev[q];
+  if (ok) return true;
   int dev = ctx->device;
-  bool ok = hipGetDevice(&dev) == hipSuccess && hipSetDevice(ctx->device) == hipSuccess;
-  for (int q = 0; q < 2 && ok; ++q) {
+  ok = hipGetDevice(&dev) == hipSuccess && hipSetDevice(ctx->device) == hipSuccess;
+  for (int q = 0; q < count && ok; ++q) {
     if (!ctx->stage[q] &&
         hipHostMalloc(&ctx->stage[q], kStageBytes, hipHostMallocDefault) != hipSuccess) {
       ctx->stage[q] = nullptr;
@@ -106,11 +108,25 @@ bool ensure_stage(cg_ctx* ctx) {
   if (!ok) (void)hipGetLastError();
   return ok;
 }
+
+// Whether a copy goes through the buffers.  They save 20 us per MB, and the
+// first use costs 0.6 to 1 ms (page-locking, the threads' stacks): a context
+// that fetches one state of 8 MB and ends should not pay for it, so copies
+// that one buffer holds take the runtime's way until they add up to the two
+// buffers' size.
+bool staged_copy(cg_ctx* ctx, size_t bytes) {
+  if (bytes > kStageBytes) return ensure_stage(ctx, 2);
+  if (!ctx->stage[0]) {
+    ctx->unstaged += bytes;
+    if (ctx->unstaged <= 2 * kStageBytes) return false;
+  }
+  return ensure_stage(ctx, 1);
+}
 }  // namespace
 
 namespace cg_host {
-// Large copies to pageable memory go through two pinned buffers in turn: while
-// one receives from the device, eight threads move the other to its place.  A
+// Large copies to pageable memory go through two pinned buffers in turn (up to
+// 16 MiB through one): while one receives from the device, eight threads move the other to its place.  A
 // host array that is written for the first time is bound by the page faults
 // of the thread that writes it (about 9 GB/s for one), not by the link.  Below
 // 4 MiB the runtime's own copy is as fast; a page-locked array gets the direct
@@ -122,7 +138,8 @@ int copy_to_host(cg_ctx* ctx, void* dst, const void* src, size_t bytes) {
   bool staged = bytes >= (4u << 20) && !runtime_memory(dst);
   if (staged) {
     lk.lock();
-    staged = ensure_stage(ctx);
+    staged = staged_copy(ctx, bytes);
+    if (!staged) lk.unlock();
   }
   if (!staged) {
     HIPCHK(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));

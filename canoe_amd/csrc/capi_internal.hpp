@@ -21,9 +21,10 @@ struct cg_ctx {
   // Device address of this device's fixed scratch array (the implicit
   // solve's entry point that allocates nothing); null if the lookup failed.
   double* fixed_scratch = nullptr;
-  // Pinned buffers of copy_to_host, allocated by its first large copy and
-  // freed with the context; one copy at a time holds them.
+  // Pinned buffers of copy_to_host, allocated when its large copies first need
+  // them and freed with the context; one copy at a time holds them.
   std::mutex stage_mu;
+  size_t unstaged = 0;  // bytes of such copies before the first buffer
   void* stage[2] = {nullptr, nullptr};
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   char err[512] = {0};

@@ -57,6 +57,7 @@ def _device_file_maps():
     return n
 
 
+# 24 bytes into an allocation: a destination inside page-locked memory
 @pytest.mark.parametrize("offset", [0, 24])
 def test_page_locked_arrays_are_written_directly(offset):
     """A download into page-locked memory, whole or inside an allocation, does
@@ -82,3 +83,36 @@ def test_page_locked_arrays_are_written_directly(offset):
         run.close()
         ctx.close()
         assert lib.hipHostFree(mem) == 0
+
+
+def test_buffers_come_when_they_pay():
+    """States of 7.6e6 B: the first four downloads of a context are the
+    runtime's own, the fifth (33.5e6 B and more in all) allocates one buffer,
+    later ones none; a large state then needs the second."""
+    ctx = ca.Context(0)
+    run, big = None, None
+    try:
+        blk, th, cfg = ca.pgen_setup(2, 64, 46, 46)
+        w = ca.pgen_init(2, 1, blk, th, cfg)
+        run = ca.Run(ctx, blk, th, cfg)
+        run.set_prim(w)
+        blk2, th2, cfg2 = ca.pgen_setup(2, 64, 128, 128)
+        w2 = ca.pgen_init(2, 2, blk2, th2, cfg2)
+        big = ca.Run(ctx, blk2, th2, cfg2)
+        big.set_prim(w2)
+        run.prim()  # and the device scratch of a download
+        grown = []
+        for r, x, b in [(run, w, blk)] * 7 + [(big, w2, blk2)]:
+            before = _device_file_maps()
+            got = r.prim()
+            grown.append((_device_file_maps() - before) >> 20)
+            sk, sj, si = b.interior()
+            np.testing.assert_array_equal(got[:, sk, sj, si], x[:, sk, sj, si])
+        print("MiB of new mappings: %s" % grown, flush=True)
+        assert grown[:3] == [0, 0, 0] and grown[3] == 16 and grown[4:7] == [0, 0, 0]
+        assert grown[7] >= 16  # the second buffer (and the larger device scratch)
+    finally:
+        for r in (run, big):
+            if r:
+                r.close()
+        ctx.close()
