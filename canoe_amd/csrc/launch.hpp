@@ -198,7 +198,10 @@ inline KLines make_lines(const KGrid& g, int dir) {
 // which they are faster, as measured at 3 to 96 levels of 1,024 to 131,072
 // lines, at the given numbers of lines; linear between these and in
 // proportion below the first; 0 is never, and above the last number of lines
-// its height counts.
+// its height counts.  Measured on states with noise of 2 m/s and 0.5 % and
+// steps at their limit, whose pivots differ from line to line; in a resting
+// state one lane per line exchanges rows less often, and the heights for 5 x 5
+// blocks are up to a third larger (a few per cent of the time at stake).
 constexpr int kEvenLines[7] = {8192, 8448, 12288, 16384, 24576, 32768, 65536};
 struct KEven {
   int h[7];
@@ -214,26 +217,27 @@ inline bool octets(const KEven& e, long long nline, int n) {
   return e.h[6] != 0 && n >= e.h[6];
 }
 // Rows: dry, with species; columns: 5 x 5, 3 x 3 blocks.
-// A stage's columns of a run, 5 x 5: 4,096 columns of 3 levels 35 us against 27
-// for one lane, of 8 45 against 49; 8,190 of 8 67 against 53, of 16 86 against
-// 95, of 64 175 against 324; 16,384 of 48 286 against 252, of 128 600 against
-// 648.  With species 12,769 of 40 274 against 258.
-constexpr KEven kRunColumns[2][2] = {{{{13, 34, 46, 90}}, {{19, 28, 57}}},
-                                     {{{10, 32, 51, 95}}, {{11, 20, 80}}}};
+// A stage's columns of a run, 5 x 5: 4,096 columns of 3 levels 36 us against 29
+// for one lane, of 8 46 against 54; 8,192 of 8 68 against 57, of 16 87 against
+// 101, of 64 184 against 352; 16,384 of 48 297 against 273, of 96 502 against
+// 529.  With species 10,240 of 24 183 against 171, of 40 262 against 270.
+constexpr KEven kRunColumns[2][2] = {{{{12, 27, 40, 67}}, {{18, 26, 51}}},
+                                     {{{9, 26, 45, 72}}, {{11, 19, 70}}}};
 // x2 / x3 lines between walls, 5 x 5 (calls of cg_implicit_solve, here and
-// below): 8,192 lines of 5 cells 92 us against 73, of 24 132 against 144, of 96 247 against 425.
-constexpr KEven kWallLines[2][2] = {{{{18, 44, 62, 70}}, {{30, 37, 56, 95}}},
-                                    {{{13, 27, 38, 49}}, {{16, 18, 33, 43}}}};
-// Periodic lines, 5 x 5: 16,384 lines of 5 cells 169 us against 98, of 48 515
-// against 840; 32,000 of 16 476 against 339, of 48 956 against 1,052.
-constexpr KEven kPeriodicLines[2][2] = {{{{7, 11, 15, 17, 24, 36}}, {{28, 33, 45, 50}}},
-                                        {{{5, 9, 11, 14, 20, 31}}, {{18, 64, 58, 56}}}};
-// x1 columns of caller arrays, 5 x 5: 262,144 columns of 5 levels 1,482 us
-// against 371, of 64 4,815 against 5,200; 65,536 of 128 2,187 against 2,712,
-// with species 2,474 against 4,750.
+// below): 8,192 lines of 5 cells 92 us against 70, of 24 131 against 154, of 96
+// 249 against 463.
+constexpr KEven kWallLines[2][2] = {{{{17, 34, 47, 60}}, {{28, 35, 53, 80}}},
+                                    {{{13, 25, 32, 42}}, {{17, 19, 28, 39}}}};
+// Periodic lines, 5 x 5: 16,384 lines of 5 cells 168 us against 100, of 48 526
+// against 853; 32,768 of 16 486 against 347, of 48 984 against 1,076.
+constexpr KEven kPeriodicLines[2][2] = {{{{7, 11, 15, 17, 24, 35}}, {{28, 33, 47, 52}}},
+                                        {{{6, 10, 13, 15, 21, 31}}, {{22, 60, 56, 54}}}};
+// x1 columns of caller arrays, 5 x 5: 131,072 columns of 5 levels 780 us
+// against 209; 65,536 of 64 1,256 against 1,431, with species 1,416 against
+// 2,435.
 constexpr KEven kCallerColumns[2][2] = {
-    {{{17, 40, 52, 54, 72, 50, 46}}, {{29, 28, 44, 60, 61, 42, 23}}},
-    {{{13, 28, 38, 39, 25, 18, 16}}, {{16, 18, 27, 40, 19, 11, 10}}}};
+    {{{13, 29, 42, 51, 63, 42, 40}}, {{20, 25, 40, 61, 61, 41, 22}}},
+    {{{14, 27, 34, 38, 25, 17, 15}}, {{19, 21, 30, 40, 20, 12, 10}}}};
 
 // Workgroups of the row kernels.
 inline unsigned rows_grid(long long nline) { return nblk(nline, RLINES * RWAVES); }

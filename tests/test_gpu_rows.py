@@ -109,8 +109,8 @@ def test_caller_periodic_lines_equal_the_oracle(ctx, flag, dims):
 # sides of the heights from which the eight-lane kernels take them, and of the
 # numbers of lines that they never take.  Walled x3 lines of moist blocks this
 # wide are refused (the shuffled species weights would lie past the end of w).
-DRY = [(10, True, (64, 17, 128)), (10, True, (64, 18, 128)), (10, True, (64, 40, 129)),
-       (2, True, (64, 29, 128)), (2, True, (64, 30, 128)),
+DRY = [(10, True, (64, 16, 128)), (10, True, (64, 17, 128)), (10, True, (64, 40, 129)),
+       (2, True, (64, 27, 128)), (2, True, (64, 28, 128)),
        (12, True, (129, 64, 6)), (4, True, (129, 64, 6)),
        (10, False, (64, 6, 128)), (10, False, (64, 7, 128)),
        (10, False, (128, 16, 128)), (10, False, (128, 17, 128)),
@@ -118,9 +118,9 @@ DRY = [(10, True, (64, 17, 128)), (10, True, (64, 18, 128)), (10, True, (64, 40,
        (2, False, (64, 27, 128)), (2, False, (64, 28, 128)),
        (2, False, (128, 5, 129)), (4, False, (129, 128, 6))]
 MOIST = [(10, True, (64, 12, 128)), (10, True, (64, 13, 128)),
-         (2, True, (64, 15, 128)), (2, True, (64, 16, 128)),
-         (10, False, (64, 4, 128)), (10, False, (64, 5, 128)),
-         (2, False, (64, 17, 128)), (2, False, (64, 18, 128)),
+         (2, True, (64, 16, 128)), (2, True, (64, 17, 128)),
+         (10, False, (64, 5, 128)), (10, False, (64, 6, 128)),
+         (2, False, (64, 21, 128)), (2, False, (64, 22, 128)),
          (12, False, (257, 128, 6)), (4, False, (129, 128, 6))]
 
 
@@ -173,10 +173,10 @@ def test_many_tall_lines_equal_the_same_lines_in_halves(ctx, flag, dims):
 
 
 @pytest.mark.parametrize("config,flag,dims", [
-    (2, 9, (16, 64, 128)), (2, 9, (17, 64, 128)), (2, 9, (5, 130, 130)), (2, 9, (53, 130, 130)),
-    (2, 1, (28, 64, 128)), (2, 1, (29, 64, 128)), (2, 1, (5, 130, 130)),
-    (4, 9, (12, 64, 128)), (4, 9, (13, 64, 128)), (4, 9, (5, 130, 130)),
-    (4, 1, (15, 64, 128)), (4, 1, (16, 64, 128)), (4, 1, (5, 130, 130))])
+    (2, 9, (12, 64, 128)), (2, 9, (13, 64, 128)), (2, 9, (5, 130, 130)), (2, 9, (52, 130, 130)),
+    (2, 1, (19, 64, 128)), (2, 1, (20, 64, 128)), (2, 1, (5, 130, 130)),
+    (4, 9, (13, 64, 128)), (4, 9, (14, 64, 128)), (4, 9, (5, 130, 130)),
+    (4, 1, (18, 64, 128)), (4, 1, (19, 64, 128)), (4, 1, (5, 130, 130))])
 @pytest.mark.parametrize("bc1", [(0, 0), (2, 2)])
 def test_caller_columns_on_both_sides_of_the_limits(ctx, config, flag, dims, bc1):
     """x1 columns of caller arrays that one or eight lanes take."""
