@@ -4,8 +4,8 @@
 // (src/snap/implicit/solve_implicit_3d.cpp:19-143,
 // periodic_forward_backward.hpp:14-232).
 //
-// One line per lane, one launch per direction (the kernels for many lines;
-// rows.hpp holds those with eight lanes per line for fewer): the blocks a_i, b_i, c_i
+// One line per lane, one launch per direction (the kernels for many or short
+// lines; rows.hpp holds those with eight lanes per line): the blocks a_i, b_i, c_i
 // and the right-hand side of each level are assembled in registers as the
 // lane climbs the line and fed straight into the recurrence; only what the
 // way back needs goes to a lane-contiguous scratch (walls: a'_i and

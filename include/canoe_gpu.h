@@ -456,7 +456,7 @@ int cg_run_block_sums(cg_run* run, int block, double* out_host);
  * segments of march_seg levels, 3D blocks only, else as 2; of march_seg's
  * default, 16, at most as many, by the size of the run); step_ms is the step
  * time measured by the autotuner.  The default column-solve shape (1, 0,
- * fused) means eight lanes per column where the run has few columns.  Dry
+ * fused) means eight lanes per column where the run has few or tall columns.  Dry
  * FP64 runs whose 32 x 8 column tiles are well filled, or are few, take all
  * faces and the divergence of their 3D blocks in one tile kernel with
  * segments of march_seg levels by the same rule; flux_block does not reach
